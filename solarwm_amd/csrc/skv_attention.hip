@@ -74,6 +74,7 @@ struct AttnArgs {
   const float* rope_hw;
   const float* rope_t;
   int gh, gw, n_qframes;
+  int rope_lds;  // 1: the kernels may stage rope_t in LDS per key frame (frames of >= 64 tokens)
   // PRoPE (camera transforms, applied after RoPE) on the same path; every matrix is a row-major
   // 4x4 acting on one group of 4 consecutive head channels:
   //   pq_t [B][n_frames][n_qframes][11][16]: W = R_k^T (P_q P_k^-1)^T R_q per temporal group
@@ -94,13 +95,13 @@ struct AttnArgs {
   // wave-uniform index reads it with a scalar load.
   int32_t flen[SKV_MAX_FRAMES];
   // Balanced key split (no mask, 8-wave groups): the n_wg workgroups share the
-  // units = B*H*n_qtiles*nt (q-tile, key tile) pairs equally; workgroup i
-  // takes units [i*units/n_wg, (i+1)*units/n_wg) in q-tile order.  A q-tile that one workgroup
+  // units = B*H*n_qtiles*nt (q-tile, key tile) pairs equally; workgroup i takes units
+  // [i*units/n_wg, (i+1)*units/n_wg) in q-tile order (share_begin).  A q-tile that one workgroup
   // covers whole is written directly; a part of a split q-tile goes to record 2i (the
   // workgroup's first segment) or 2i+1 (its last) of part_o / part_ml, and attn_combine_kernel
   // merges the records of each split q-tile.
   int split;
-  int64_t units;
+  int share_base, share_rem;  // units / n_wg and units % n_wg
   // q-tile (in (b, h)-major order) that unit 0 / workgroup 0 of this grid starts at: 0, except
   // for the tail launch of a grid whose last round is split (the full rounds run unsplit first)
   int qt_base;
@@ -114,6 +115,32 @@ struct AttnArgs {
   int32_t seg_nf[SKV_MAX_SEGMENTS];
 };
 
+// First unit of workgroup i's share, floor(i * units / n_wg) (AttnArgs.split), in 32 bits: as 64-bit
+// divisions the bounds took some 600 instructions at the start of every workgroup.
+__device__ inline int share_begin(const AttnArgs& a, int i) {
+  return i * a.share_base + (int)((uint32_t)(i * a.share_rem) / (uint32_t)a.n_wg);
+}
+
+// The launch's arguments as one segment of a split share sees them.  The segment loop of the
+// SPLIT instances reads them through an opaque copy of the kernel-argument pointer: otherwise
+// every argument-derived value is hoisted out of the loop and stays live through the tile loop
+// (29-47 SGPRs of the bf16 instances spilled to VGPR lanes that way, and were read back with
+// v_readlane on the tile path; with the copy none spills, which leaves the frame-aligned
+// instances room for the four-buffer ring: H24 x 2640 queries over 21 x 880 keys with RoPE 619 ->
+// 601 us a layer pass, H12 x 1170 over 8190 float32 keys 183 -> 177).
+template <bool SPLIT>
+__device__ inline const AttnArgs& segment_args(const AttnArgs& args) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  if constexpr (SPLIT) {
+    typedef const __attribute__((address_space(4))) AttnArgs* args_p;
+    args_p p = (args_p)__builtin_amdgcn_kernarg_segment_ptr();  // the kernels' only parameter
+    asm volatile("" : "+s"(p));
+    return *(const AttnArgs*)p;
+  }
+#endif
+  return args;
+}
+
 // Wan's split of a head's 64 complex channel pairs (2i, 2i+1): 22 temporal, 21 height, 21 width
 // (causal_model.py:1855-1866).
 constexpr int kRopeT = 22, kRopeHW = 21;
@@ -124,6 +151,14 @@ constexpr int kWPair = kGroupsT * 16 * 4;  // bytes of W per (query frame, key f
 constexpr int kWMaxQF = 5;
 constexpr int kWBuf = 4096;                // >= kWMaxQF * kWPair, whole 1 KB wave chunks
 static_assert(kWMaxQF * kWPair <= kWBuf, "W buffer too small");
+// RoPE on load: the temporal angles (22 pairs x cos, sin = 176 B) of the q-tile's query frames (at
+// most 5 when frame_tokens >= 64) against the key frame a tile opens are staged in LDS, one table
+// slot per ring buffer, with the K tile that opens the frame.
+constexpr int kTabSlot = 1024;
+constexpr int kTabFrames = 5;
+static_assert(kTabFrames * 8 * kRopeT <= kTabSlot && kTabFrames * 11 <= 64,
+              "one 64-lane DMA of 16 B pieces fills a table slot");
+static_assert((256 - 1) / 64 + 2 <= kTabFrames, "256 rows of >= 64-token frames span <= 5 frames");
 
 // y[4g .. 4g+4) <- m (row-major 4x4) x y[4g .. 4g+4)
 __device__ inline void xform4(Vec8<float>& y, int g, const float* m) {
@@ -146,6 +181,9 @@ constexpr int kTileBytes = 32 * kBlockBytes;  // K (16 KB) + V^T (16 KB)
 
 typedef __attribute__((address_space(3))) void lds_void_t;
 typedef __attribute__((address_space(1))) void glb_void_t;
+// vector loads from caller tables that are only known to be float-aligned
+typedef float f32x2_u __attribute__((ext_vector_type(2), aligned(4)));
+typedef float f32x4_u __attribute__((ext_vector_type(4), aligned(4)));
 
 // Row m of a 32-row MFMA block reads key key_perm(m) of the block.  With the 32x32 C layout
 // (lane l, register i -> row (i/4)*8 + (l/32)*4 + i%4) this puts key (i/8)*16 + (l/32)*8 + i%8
@@ -526,19 +564,20 @@ __device__ inline void mask_tile(f32x16 (&s)[2], int hh, int tok0, int T, int ke
 
 // K and V^T tile buffers of attn_kernel's ring: 4 (a barrier every second step) for 8-wave groups
 // over 2-byte pools, 2 otherwise: 4-wave groups run two workgroups per CU, whose 2 x 128 KB would
-// not fit the 160 KB of LDS; fp32 pools and the frame-aligned split spill registers with the
-// longer ring.
-constexpr int attn_ring(int nw, int rm, int kt_bytes, bool split, bool pk) {
-  return nw == 8 && kt_bytes == 2 && (pk || !split) ? 4 : 2;
-}
+// not fit the 160 KB of LDS; fp32 and fp8 pools stage through registers, which the longer ring
+// would spill.
+constexpr int attn_ring(int nw, int kt_bytes) { return nw == 8 && kt_bytes == 2 ? 4 : 2; }
 // PRoPE matrix buffers: one per key frame in flight (frame j in buffer j mod n); with the longer
 // ring a frame's matrices are staged three steps before use, so frames of a single tile need four
 constexpr int attn_wbufs(int ring) { return ring == 4 ? 4 : 2; }
-constexpr size_t attn_lds_bytes(int nw, int rm, int kt_bytes, bool split, bool pk) {
-  return (size_t)attn_ring(nw, rm, kt_bytes, split, pk) * kTileBytes +
-         (rm == 2 ? (size_t)attn_wbufs(attn_ring(nw, rm, kt_bytes, split, pk)) * kWBuf : 0);
+constexpr size_t attn_lds_bytes(int nw, int rm, int kt_bytes) {
+  return (size_t)attn_ring(nw, kt_bytes) * kTileBytes +
+         (rm == 2 ? (size_t)attn_wbufs(attn_ring(nw, kt_bytes)) * kWBuf : 0) +
+         (rm == 1 && kt_bytes == 2 ? (size_t)attn_ring(nw, kt_bytes) * kTabSlot : 0);
 }
 
+// RM: 0 = Q as given, 1 = RoPE on load, 2 = RoPE + PRoPE, 3 = RoPE on load over frames of fewer than
+// 64 tokens.
 // PK: key tiles packed across frame boundaries (PackedWalk; whole frames of T = 8k tokens, 2-byte
 // pools, no RoPE): a window of n frames takes ceil(n T / 64) tiles instead of n ceil(T / 64).
 // SEG: the grid's q-tiles belong to consecutive query segments, each over its own slice of the
@@ -546,18 +585,21 @@ constexpr size_t attn_lds_bytes(int nw, int rm, int kt_bytes, bool split, bool p
 template <int NW, typename QT, typename KT, int RM, bool SPLIT = false, bool PK = false,
           bool SEG = false>
 __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
-void attn_kernel(AttnArgs a) {
+void attn_kernel(AttnArgs args) {
   static_assert(!PK || (RM == 0 && sizeof(KT) == 2), "packed tiles: 2-byte pools, no RoPE");
   static_assert(!SEG || (RM == 0 && !SPLIT), "segments: no RoPE, no split");
   constexpr int kBQ = NW * 32;
   // LDS map: kRing K buffers, then kRing V^T buffers (tile x in buffer x mod kRing), then (PRoPE)
   // kWN matrix buffers.  A step reads K(tau+1) and V(tau-1) and loads K(tau+kL+1) and V(tau+kL-1);
   // the workgroup meets at a barrier after every kL-th step.  kL = 1 (two buffers each) for
-  // 4-wave groups (two workgroups share a CU's LDS), fp32 pools and the frame-aligned split;
-  // the others take kL = 2.
-  constexpr int kRing = attn_ring(NW, RM, (int)sizeof(KT), SPLIT, PK);
+  // 4-wave groups (two workgroups share a CU's LDS) and register-staged pools; the others take
+  // kL = 2.
+  constexpr int kRing = attn_ring(NW, (int)sizeof(KT));
   constexpr int kL = kRing / 2;
   constexpr int kWN = attn_wbufs(kRing);
+  // RoPE on load: the temporal angles come from LDS (RM = 1 over 2-byte pools) or, for frames under
+  // 64 tokens, straight from memory (RM = 3, and RM = 1 over fp8 pools)
+  constexpr bool kRopeLds = RM == 1 && sizeof(KT) == 2;
   using ET = typename OpOf<KT>::E;     // MFMA operand element
   using etx8 = typename OpOf<KT>::x8;
   // LDS: K tiles in [0, 32 KB) (two buffers), V^T tiles in [32 KB, 64 KB) (two buffers).
@@ -570,7 +612,7 @@ void attn_kernel(AttnArgs a) {
   int logical;
   {
     const int bid = blockIdx.x, xcd = bid & 7, idx = bid >> 3;
-    const int per = a.n_wg >> 3, rem = a.n_wg & 7;
+    const int per = args.n_wg >> 3, rem = args.n_wg & 7;
     logical = xcd * per + min(xcd, rem) + idx;
   }
   // Segments: key tiles [tb, te) of q-tile qg; one whole q-tile unless split.  A split share
@@ -578,24 +620,25 @@ void attn_kernel(AttnArgs a) {
   // whole ones run first, then the last segment (key tiles from 0, in step with the other
   // workgroups, which all start at key tile 0), then the first (the tail of a q-tile, a fixed
   // number of tiles ahead of them): K/V tiles stay shared through L2 as in the unsplit grid.
-  const int nt = a.nt;
+  const int nt = args.nt;
   int q_first = logical, nseg = 1;
-  int64_t u0 = 0, u1 = 0;
+  int u0 = 0, u1 = 0;
   if constexpr (SPLIT) {
-    u0 = (int64_t)logical * a.units / a.n_wg;
-    u1 = (int64_t)(logical + 1) * a.units / a.n_wg;
-    q_first = (int)(u0 / nt);
-    nseg = u1 > u0 ? (int)((u1 - 1) / nt) - q_first + 1 : 0;
+    u0 = share_begin(args, logical);
+    u1 = share_begin(args, logical + 1);
+    q_first = u0 / nt;
+    nseg = u1 > u0 ? (u1 - 1) / nt - q_first + 1 : 0;
   }
   for (int k = 0; k < nseg; ++k) {
   const int seg = nseg == 1 ? 0 : k < nseg - 2 ? k + 1 : k == nseg - 2 ? nseg - 1 : 0;
   const int qg = q_first + seg;
   int tb = 0, te = nt;
   if constexpr (SPLIT) {
-    if (seg == 0) tb = (int)(u0 - (int64_t)q_first * nt);
-    if (seg == nseg - 1) te = (int)(u1 - (int64_t)qg * nt);
+    if (seg == 0) tb = u0 - q_first * nt;
+    if (seg == nseg - 1) te = u1 - qg * nt;
   }
   if (k > 0) __syncthreads();  // the previous segment's last LDS reads are done
+  const AttnArgs& a = segment_args<SPLIT>(args);
   const int qt = (qg + a.qt_base) % a.n_qtiles;
   const int bh = (qg + a.qt_base) / a.n_qtiles;
   const int h = bh % a.H, b = bh / a.H;
@@ -629,69 +672,120 @@ void attn_kernel(AttnArgs a) {
 
   // Q^T operand: lane (n, hh) holds q[qrow][k*16 + hh*8 .. +7] for k = 0..7.
   etx8 qf[8];
-  // RM = 0: Q as given.  RM = 1 (RoPE): the query's height/width pairs are rotated once here;
+  // RM = 0: Q as given.  RM = 1 (RoPE): the query's height/width pairs are rotated once at load;
   // its temporal pairs (0..21, in qf[0..2]) are kept unrotated in qt0 and turned by
   // (p_query - p_key) per key frame below.  RM = 2 (RoPE + PRoPE): as RM = 1, the spatial
   // groups then take P_q^T, and the temporal groups take the per-key-frame matrix W below.
   [[maybe_unused]] etx8 qt0[3];
+  // Every global load of the query (the row, its RoPE angles, its P_q^T) is issued here, without a
+  // branch on the lane, before the tile loads below and long before its first use: with the loads
+  // behind lane-dependent branches (rows past the end, pairs that are temporal for one half of the
+  // wave only) the RoPE / PRoPE instances waited out some thirty L2 round trips one by one at the
+  // start of every q-tile (with the matrices read from LDS below: 30 layers of H24, 1215 queries
+  // over 18 x 405 keys, fused PRoPE, 5.74 -> 5.38 ms).  Rows past the end load the last row's, then count as zeros (their
+  // products then toggle few bits: at full chip the clock is power-limited).
+  const int qrc = min(qrow, qend - 1);
   [[maybe_unused]] int qfi = 0;  // query frame of this lane's row
+  Vec8<QT> qx[8];
+  // angles of pairs 16 + 8 k + 4 hh + m (pairs below 22 are temporal: an entry nobody uses)
+  [[maybe_unused]] f32x2_u qhw[6][4];
+  [[maybe_unused]] f32x4 qps[4];  // P_q^T of the row's frame, by rows
+  const float* qw = a.q_w + h * kHeadDim + hh * 8;
   {
     const QT* qp = static_cast<const QT*>(a.q) + (int64_t)b * a.q_sb + (int64_t)h * a.q_sh +
-                   (int64_t)(qlive ? qrow : 0) * a.q_st + hh * 8;
-    // RMSNorm factor of this row (0 for dead rows) and its channel weights
-    const float qn = a.q_rms && qlive ? a.q_rms[(int64_t)b * a.q_rms_sb + qrow] : 0.f;
-    const float* qw = a.q_w + h * kHeadDim + hh * 8;
+                   (int64_t)qrc * a.q_st + hh * 8;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) qx[k] = Vec8<QT>::load(qp + k * 16);
     if constexpr (RM > 0) {
-      const int qr = qlive ? qrow : a.Lq - 1;
-      qfi = qr / a.T;
-      const int tt = qr - qfi * a.T, hq = tt / a.gw, wq = tt - hq * a.gw;
+      qfi = qrc / a.T;
+      const int tt = qrc - qfi * a.T, hq = tt / a.gw, wq = tt - hq * a.gw;
 #pragma unroll
-      for (int k = 0; k < 8; ++k) {
-        const Vec8<QT> x = qlive ? Vec8<QT>::load(qp + k * 16) : Vec8<QT>::zero();
-        Vec8<float> y;
-        if (a.q_rms) {
-#pragma unroll
-          for (int e = 0; e < 8; ++e) y.set(e, (float)x.get(e) * qn * qw[k * 16 + e]);
-        } else {
-#pragma unroll
-          for (int e = 0; e < 8; ++e) y.set(e, (float)(bf16)x.get(e));
-        }
+      for (int k = 0; k < 6; ++k)
 #pragma unroll
         for (int m = 0; m < 4; ++m) {
-          const int pr = k * 8 + hh * 4 + m;
-          if (pr < kRopeT) continue;
-          const int idx = pr < kRopeT + kRopeHW ? hq * kRopeHW + (pr - kRopeT)
+          const int pr = 16 + 8 * k + 4 * hh + m;
+          const int idx = pr < kRopeT + kRopeHW ? hq * kRopeHW + max(pr - kRopeT, 0)
                                                 : (a.gh + wq) * kRopeHW + (pr - kRopeT - kRopeHW);
-          const float c = a.rope_hw[2 * idx], sn = a.rope_hw[2 * idx + 1];
-          const float u = y.get(2 * m), v = y.get(2 * m + 1);
-          y.set(2 * m, u * c - v * sn);
-          y.set(2 * m + 1, u * sn + v * c);
+          qhw[k][m] = *reinterpret_cast<const f32x2_u*>(a.rope_hw + 2 * idx);
         }
-        if constexpr (RM == 2) {
-          const float* ps = a.pq_s + ((int64_t)b * a.n_qframes + qfi) * 16;
+    }
+    if constexpr (RM == 2) {
+      const float* ps = a.pq_s + ((int64_t)b * a.n_qframes + qfi) * 16;
 #pragma unroll
-          for (int gg = 0; gg < 2; ++gg)
-            if (4 * k + 2 * hh + gg >= kGroupsT) xform4(y, gg, ps);
-        }
-        qf[k] = OpOf<KT>::from(y);
-      }
-#pragma unroll
-      for (int k = 0; k < 3; ++k) qt0[k] = qf[k];
-    } else if (a.q_rms) {
-#pragma unroll
-      for (int k = 0; k < 8; ++k) {
-        const Vec8<QT> x = qlive ? Vec8<QT>::load(qp + k * 16) : Vec8<QT>::zero();
-        Vec8<float> y;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) y.set(e, (float)x.get(e) * qn * qw[k * 16 + e]);
-        qf[k] = OpOf<KT>::from(y);
-      }
-    } else {
-#pragma unroll
-      for (int k = 0; k < 8; ++k)
-        qf[k] = OpOf<KT>::from(qlive ? Vec8<QT>::load(qp + k * 16) : Vec8<QT>::zero());
+      for (int i = 0; i < 4; ++i) qps[i] = *reinterpret_cast<const f32x4_u*>(ps + 4 * i);
     }
   }
+  // qx -> qf (and qt0), once the tile loads are in flight
+  auto form_q = [&]() __attribute__((always_inline)) {
+    Vec8<float> y[8];
+    if (a.q_rms) {  // RMSNorm factor of this row and its channel weights
+      const float qn = a.q_rms[(int64_t)b * a.q_rms_sb + qrc];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        const Vec8<float> wk = Vec8<float>::load(qw + k * 16);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) y[k].set(e, (float)qx[k].get(e) * qn * wk.get(e));
+      }
+    } else if constexpr (RM > 0) {
+#pragma unroll
+      for (int k = 0; k < 8; ++k)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) y[k].set(e, (float)(bf16)qx[k].get(e));
+    } else {
+#pragma unroll
+      for (int k = 0; k < 8; ++k) qf[k] = OpOf<KT>::from(qlive ? qx[k] : Vec8<QT>::zero());
+      return;
+    }
+    if constexpr (RM > 0) {
+#pragma unroll
+      for (int k = 2; k < 8; ++k) {
+#pragma unroll
+        for (int m = 0; m < 4; ++m) {
+          const bool spatial = k * 8 + hh * 4 + m >= kRopeT;
+          const float c = qhw[k - 2][m][0], sn = qhw[k - 2][m][1];
+          const float u = y[k].get(2 * m), v = y[k].get(2 * m + 1);
+          const float u2 = u * c - v * sn, v2 = u * sn + v * c;
+          y[k].set(2 * m, spatial ? u2 : u);
+          y[k].set(2 * m + 1, spatial ? v2 : v);
+        }
+        if constexpr (RM == 2) {
+          float ps[16];
+#pragma unroll
+          for (int i = 0; i < 16; ++i) ps[i] = qps[i >> 2][i & 3];
+          Vec8<float> z = y[k];
+          xform4(z, 0, ps);
+          xform4(z, 1, ps);
+#pragma unroll
+          for (int e = 0; e < 8; ++e)
+            if (4 * k + 2 * hh + (e >> 2) >= kGroupsT) y[k].set(e, z.get(e));
+        }
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < 8; ++k) qf[k] = OpOf<KT>::from(qlive ? y[k] : Vec8<float>::zero());
+    if constexpr (RM > 0) {
+#pragma unroll
+      for (int k = 0; k < 3; ++k) qt0[k] = qf[k];
+    }
+  };
+  // RoPE: the angles of the q-tile's query frames qf_lo .. against key frame j -> the table slot of
+  // the tile x that opens frame j (slot x mod kRing, written with K(x) and read before QK(x), so it
+  // lives like K(x)'s buffer).  Lane i of wave 0 moves 16 bytes: pairs 2 (i % 11) .. +1 of query
+  // frame qf_lo + i / 11; lanes past the q-tile's frames repeat frame qf_lo's pieces into the
+  // slot's unread tail.
+  [[maybe_unused]] auto stage_tab = [&](int x, int j) __attribute__((always_inline)) {
+#if defined(__HIP_DEVICE_COMPILE__)  // the host pass would drop the calling kernels' launch stubs
+    if constexpr (RM == 1) {
+      const int lo = q0 / a.T, count = (min(q0 + kBQ, a.Lq) - 1) / a.T - lo + 1;
+      const int f = lane / 11, pp = lane - 11 * f;
+      const __amdgpu_buffer_rsrc_t r =
+          __builtin_amdgcn_make_buffer_rsrc((void*)a.rope_t, (short)0, 0x7fffffff, 0x00020000);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          r, (lds_void_t*)(lds + kRing * kTileBytes + (x & (kRing - 1)) * kTabSlot), 16,
+          (uint32_t)((((lo + (f < count ? f : 0)) * a.n_frames + j) * kRopeT + 2 * pp) * 8), 0, 0, 0);
+    }
+#endif
+  };
   // PRoPE: W of key frame j for query frames [qf_lo, qf_lo + count) -> LDS buffer j & 1 (waves
   // 0..3 move 1 KB each with direct global->LDS loads; completion is awaited with the tiles')
   [[maybe_unused]] const int qf_lo = q0 / a.T;
@@ -710,51 +804,80 @@ void attn_kernel(AttnArgs a) {
   };
   // qf[0..2] <- qt0 with the temporal pairs turned by the angle of (query frame, key frame j)
   // (RM = 1), or with each temporal group multiplied by that pair's W (RM = 2)
-  [[maybe_unused]] auto rot_q = [&](int j) {
+  [[maybe_unused]] auto rot_q = [&](int x, int j) {
     if constexpr (RM == 2) {
-      // W of (this lane's query frame, key frame j), staged in LDS by issue_w; one group's
-      // rows are live at a time (this runs inside the main loop, where registers are scarce)
-      const float* wt = reinterpret_cast<const float*>(lds + kRing * kTileBytes + (j % kWN) * kWBuf) +
-                        (qfi - qf_lo) * (kGroupsT * 16);
+      // W of (this lane's query frame, key frame j), staged in LDS by issue_w, read by asm blocks
+      // of one group (4 rows) each: the compiler's own LDS reads of a DMA-written buffer would
+      // first wait for every DMA in flight (the next tiles' K and V), which the barrier after W's
+      // DMA already covers.  The half of the wave whose last group is spatial reads group 10 again
+      // (in bounds) and keeps its channels.
+      const uint32_t wt = (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) char*)(
+          lds + kRing * kTileBytes + (j % kWN) * kWBuf + (qfi - qf_lo) * kWPair);
 #pragma unroll
       for (int k = 0; k < 3; ++k) {
 #pragma unroll
         for (int gg = 0; gg < 2; ++gg) {
           const int g = 4 * k + 2 * hh + gg;
-          if (g >= kGroupsT) continue;
+          const bool live = g < kGroupsT;
+          f32x4 m[4];
+          asm volatile("ds_read_b128 %0, %4\n\tds_read_b128 %1, %4 offset:16\n\t"
+                       "ds_read_b128 %2, %4 offset:32\n\tds_read_b128 %3, %4 offset:48\n\t"
+                       "s_waitcnt lgkmcnt(0)"
+                       : "=&v"(m[0]), "=&v"(m[1]), "=&v"(m[2]), "=&v"(m[3])
+                       : "v"(wt + 64u * (uint32_t)min(g, kGroupsT - 1))
+                       : "memory");
           // an opaque copy keeps the loop-invariant bf16 -> fp32 conversion here instead of
           // hoisted out of the main loop (24 live floats there would spill)
           bf16x8 t = qt0[k];
           asm volatile("" : "+v"(t));
-          float x[4], r[4];
+          float x[4];
 #pragma unroll
           for (int e = 0; e < 4; ++e) x[e] = (float)t[4 * gg + e];
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
-            const float4 m = *reinterpret_cast<const float4*>(wt + g * 16 + 4 * i);
-            r[i] = fmaf(m.x, x[0], fmaf(m.y, x[1], fmaf(m.z, x[2], m.w * x[3])));
+            const float r = fmaf(m[i][0], x[0], fmaf(m[i][1], x[1], fmaf(m[i][2], x[2], m[i][3] * x[3])));
+            qf[k][4 * gg + i] = live ? (bf16)r : t[4 * gg + i];
           }
-#pragma unroll
-          for (int e = 0; e < 4; ++e) qf[k][4 * gg + e] = (bf16)r[e];
-          asm volatile("" ::: "memory");
         }
       }
       return;
     }
-    const float* tb = a.rope_t + ((int64_t)qfi * a.n_frames + j) * (2 * kRopeT);
+    // cos, sin of pairs 8 k + 4 hh .. +3 of (query frame, key frame j); the second half of the
+    // wave reads pairs 22 and 23 of k = 2 too (in bounds of the slot: <= 4 * 176 + 192) and keeps
+    // those channels
+    f32x4 tq[6];
+    if constexpr (kRopeLds) {  // the slot of tile x, read by an asm block for the reason given above
+      const uint32_t tab = (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) char*)(
+          lds + kRing * kTileBytes + (x & (kRing - 1)) * kTabSlot +
+          (qfi - q0 / a.T) * (8 * kRopeT) + hh * 32);
+      asm volatile("ds_read_b128 %0, %6\n\tds_read_b128 %1, %6 offset:16\n\t"
+                   "ds_read_b128 %2, %6 offset:64\n\tds_read_b128 %3, %6 offset:80\n\t"
+                   "ds_read_b128 %4, %6 offset:128\n\tds_read_b128 %5, %6 offset:144\n\t"
+                   "s_waitcnt lgkmcnt(0)"
+                   : "=&v"(tq[0]), "=&v"(tq[1]), "=&v"(tq[2]), "=&v"(tq[3]), "=&v"(tq[4]), "=&v"(tq[5])
+                   : "v"(tab)
+                   : "memory");
+    } else {
+      const float* tb = a.rope_t + ((int64_t)qfi * a.n_frames + j) * (2 * kRopeT) + hh * 8;
+#pragma unroll
+      for (int i = 0; i < 6; ++i)  // the last piece of the second half lies past the 22 pairs
+        tq[i] = *reinterpret_cast<const f32x4_u*>(tb + (i == 5 && hh ? 0 : (i >> 1) * 16 + (i & 1) * 4));
+    }
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
+      etx8 t = qt0[k];  // opaque, as above
+      asm volatile("" : "+v"(t));
       Vec8<float> y;
 #pragma unroll
-      for (int e = 0; e < 8; ++e) y.set(e, (float)qt0[k][e]);
+      for (int e = 0; e < 8; ++e) y.set(e, (float)t[e]);
 #pragma unroll
       for (int m = 0; m < 4; ++m) {
-        const int pr = k * 8 + hh * 4 + m;
-        if (pr >= kRopeT) continue;
-        const float c = tb[2 * pr], sn = tb[2 * pr + 1];
+        const bool temporal = k * 8 + hh * 4 + m < kRopeT;
+        const float c = tq[2 * k + (m >> 1)][2 * (m & 1)], sn = tq[2 * k + (m >> 1)][2 * (m & 1) + 1];
         const float u = y.get(2 * m), v = y.get(2 * m + 1);
-        y.set(2 * m, u * c - v * sn);
-        y.set(2 * m + 1, u * sn + v * c);
+        const float u2 = u * c - v * sn, v2 = u * sn + v * c;
+        y.set(2 * m, temporal ? u2 : u);
+        y.set(2 * m + 1, temporal ? v2 : v);
       }
       qf[k] = OpOf<KT>::from(y);
     }
@@ -887,12 +1010,22 @@ void attn_kernel(AttnArgs a) {
       for (int x = 1; x <= kL; ++x)
         if (ntau > x && (tb + x) % a.ntiles_f == 0) issue_w((tb + x) / a.ntiles_f);
     }
+    if constexpr (RM == 1) {
+      // likewise the angles of those frames
+      if (kRopeLds && loader.wu == 0) {
+        stage_tab(0, tb / a.ntiles_f);
+#pragma unroll
+        for (int x = 1; x <= kL; ++x)
+          if (ntau > x && (tb + x) % a.ntiles_f == 0) stage_tab(x, (tb + x) / a.ntiles_f);
+      }
+    }
+    form_q();
 #pragma unroll
     for (int r = 0; r < 16 / NW; ++r)
       *reinterpret_cast<bf16x8*>(vb_lds(-1) + (tid + NW * 64 * r) * 16) = Vec8<bf16>::zero().to_bf16();
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
-    if constexpr (RM > 0) rot_q(tb / a.ntiles_f);
+    if constexpr (RM > 0) rot_q(0, tb / a.ntiles_f);
     qk_tile(kb_lds(0) + lane16, qf, s_cur);
     if constexpr (PK) {
       const int key0 = tb * kTile;  // packed tiles hold no padding keys: only the limit masks
@@ -991,9 +1124,12 @@ void attn_kernel(AttnArgs a) {
       // W for the frame tile tau+kL+1 opens (rot_q reads it at the start of step tau+kL)
       if (tau + kL + 1 < ntau && kw.t == 0) issue_w(kw.j);
     }
+    if constexpr (RM == 1) {  // the angles of the frame that tile tau+kL+1 opens travel with its K
+      if (kRopeLds && loader.wu == 0 && tau + kL + 1 < ntau && kw.t == 0) stage_tab(tau + kL + 1, kw.j);
+    }
     if constexpr (RM > 0) {
       // QK(tau+1) below opens a new key frame: turn Q's temporal pairs for it
-      if (tau + 1 < ntau && mw.t == 0) rot_q(mw.j);
+      if (tau + 1 < ntau && mw.t == 0) rot_q(tau + 1, mw.j);
     }
     if constexpr (RM == 2) {
 #pragma unroll
@@ -1144,6 +1280,7 @@ void attn_kernel(AttnArgs a) {
   static_assert(kL == 1 || kL == 2, "the barrier test above assumes kL <= 2 (cb = tau & 1)");
   int tau = 0;
   for (; tau + 1 < ntau; tau += 2) {
+
     step(tau, 0, sA, sB, pA, pB);
     step(tau + 1, 1, sB, sA, pB, pA);
   }
@@ -1190,8 +1327,12 @@ void attn_kernel(AttnArgs a) {
     QT* op = static_cast<QT*>(a.o) + (int64_t)b * a.o_sb + (int64_t)h * a.o_sh +
              (int64_t)qrow * a.o_st;
     // lane (n, hh) holds channels db*32 + g*8 + hh*4 .. +3 of its query: whole PRoPE groups
-    [[maybe_unused]] const float* po = nullptr;
-    if constexpr (RM == 2) po = a.pq_o + ((int64_t)b * a.n_qframes + qfi) * 16;
+    [[maybe_unused]] float po[16];  // P_q, loaded once (the stores below might alias it)
+    if constexpr (RM == 2) {
+      const float* pm = a.pq_o + ((int64_t)b * a.n_qframes + qfi) * 16;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) po[i] = pm[i];
+    }
 #pragma unroll
     for (int db = 0; db < 4; ++db)
 #pragma unroll
@@ -1251,14 +1392,9 @@ constexpr int fp8_ring(int nw) { return nw == 8 ? 4 : 2; }
 // one table slot per ring buffer: the temporal angles (22 pairs x cos, sin = 176 B) of the
 // q-tile's query frames (at most 5) against the key frame a tile opens
 constexpr int kFp8QRows = 4096;
-constexpr int kFp8TabSlot = 1024;
-constexpr int kFp8TabFrames = 5;
-static_assert(kFp8TabFrames * 8 * kRopeT <= kFp8TabSlot && kFp8TabFrames * 11 <= 64,
-              "one 64-lane DMA of 16 B pieces fills a table slot");
-static_assert((256 - 1) / 64 + 2 <= kFp8TabFrames, "256 rows of >= 64-token frames span <= 5 frames");
 constexpr int fp8_lds_bytes(int nw, int rm = 0) {
   return 2 * fp8_ring(nw) * 4 * kOp8 +
-         (rm == 1 ? nw * kFp8QRows + fp8_ring(nw) * kFp8TabSlot : 0);
+         (rm == 1 ? nw * kFp8QRows + fp8_ring(nw) * kTabSlot : 0);
 }
 typedef int i32x8 __attribute__((ext_vector_type(8)));
 
@@ -1351,7 +1487,7 @@ __device__ inline void qk64(const char* kl, const i32x8 (&q8)[2], const f32x16& 
 // row scale bounds every rotation: max(spatial |q|, temporal pair norms) / 448.
 template <int NW, typename QT, bool SPLIT = false, int RM = 0>
 __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
-void attn_fp8_kernel(AttnArgs a) {
+void attn_fp8_kernel(AttnArgs args) {
   static_assert(RM == 0 || RM == 1, "fp8 MFMA attention: no RoPE or RoPE on load");
   constexpr int kBQ = NW * 32;
   constexpr int kDma = 16 / NW;     // 1 KB DMA parts per wave per tile (8 for K, 8 for V^T)
@@ -1360,29 +1496,30 @@ void attn_fp8_kernel(AttnArgs a) {
   int logical;
   {
     const int bid = blockIdx.x, xcd = bid & 7, idx = bid >> 3;
-    const int per = a.n_wg >> 3, rem = a.n_wg & 7;
+    const int per = args.n_wg >> 3, rem = args.n_wg & 7;
     logical = xcd * per + min(xcd, rem) + idx;
   }
   // Segments: key tiles [tb, te) of q-tile qg, as in attn_kernel (one whole q-tile unless split;
   // a split share runs its whole q-tiles, then its last segment, then its first).
-  const int nt = a.nt;
+  const int nt = args.nt;
   int q_first = logical, nseg = 1;
-  int64_t u0 = 0, u1 = 0;
+  int u0 = 0, u1 = 0;
   if constexpr (SPLIT) {
-    u0 = (int64_t)logical * a.units / a.n_wg;
-    u1 = (int64_t)(logical + 1) * a.units / a.n_wg;
-    q_first = (int)(u0 / nt);
-    nseg = u1 > u0 ? (int)((u1 - 1) / nt) - q_first + 1 : 0;
+    u0 = share_begin(args, logical);
+    u1 = share_begin(args, logical + 1);
+    q_first = u0 / nt;
+    nseg = u1 > u0 ? (u1 - 1) / nt - q_first + 1 : 0;
   }
   for (int k = 0; k < nseg; ++k) {
   const int seg = nseg == 1 ? 0 : k < nseg - 2 ? k + 1 : k == nseg - 2 ? nseg - 1 : 0;
   const int qg = q_first + seg;
   int tb = 0, te = nt;
   if constexpr (SPLIT) {
-    if (seg == 0) tb = (int)(u0 - (int64_t)q_first * nt);
-    if (seg == nseg - 1) te = (int)(u1 - (int64_t)qg * nt);
+    if (seg == 0) tb = u0 - q_first * nt;
+    if (seg == nseg - 1) te = u1 - qg * nt;
   }
   if (k > 0) __syncthreads();  // the previous segment's last LDS reads are done
+  const AttnArgs& a = segment_args<SPLIT>(args);
   const int qt = (qg + a.qt_base) % a.n_qtiles;
   const int bh = (qg + a.qt_base) / a.n_qtiles;
   const int h = bh % a.H, b = bh / a.H;
@@ -1396,87 +1533,109 @@ void attn_fp8_kernel(AttnArgs a) {
   const int qrow = q0 + w * 32 + n;
   const bool qlive = qrow < a.Lq;
 
-  // Q row quantisation: lane (n, hh) holds channels cs*64 + 32 hh .. +31 for cs = 0, 1.
+  // Q row quantisation: lane (n, hh) holds channels cs*64 + 32 hh .. +31 for cs = 0, 1.  The row and
+  // its angles are loaded here, without a branch on the lane (rows past the end load the last
+  // row's and count as zeros), and quantised (form_q) once the first tiles' loads are in flight.
   i32x8 q8[2];
-  float q_scale;
+  float q_scale = 0.f;
   [[maybe_unused]] int qfi = 0;        // RM = 1: query frame of this lane's row
   [[maybe_unused]] float q_inv = 0.f;  // RM = 1: 448 / the row's bound
+  const int qrc = min(qrow, a.Lq - 1);
+  Vec8<QT> qx[8];
+  [[maybe_unused]] f32x2_u qhw[2][16];  // cos, sin of pair cs * 32 + 16 hh + m (spatial pairs)
+  const float* qw = a.q_w + h * kHeadDim + hh * 32;
   {
-    float qv[64];  // qv[cs * 32 + j] = channel cs * 64 + 32 hh + j
     const QT* qp = static_cast<const QT*>(a.q) + (int64_t)b * a.q_sb + (int64_t)h * a.q_sh +
-                   (int64_t)(qlive ? qrow : 0) * a.q_st + hh * 32;
-    const float qn = a.q_rms && qlive ? a.q_rms[(int64_t)b * a.q_rms_sb + qrow] : 0.f;
-    const float* qw = a.q_w + h * kHeadDim + hh * 32;
+                   (int64_t)qrc * a.q_st + hh * 32;
 #pragma unroll
-    for (int cs = 0; cs < 2; ++cs)
-#pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        Vec8<QT> v = qlive ? Vec8<QT>::load(qp + cs * 64 + c * 8) : Vec8<QT>::zero();
-        if (a.q_rms) {  // normalised Q in bf16, as the reference's norm_q output
-#pragma unroll
-          for (int j = 0; j < 8; ++j)
-            qv[cs * 32 + c * 8 + j] = (float)(bf16)((float)v.get(j) * qn * qw[cs * 64 + c * 8 + j]);
-        } else {
-#pragma unroll
-          for (int j = 0; j < 8; ++j) qv[cs * 32 + c * 8 + j] = (float)(bf16)v.get(j);  // bf16 first
-        }
-      }
-    float amax = 0.f;
+    for (int i = 0; i < 8; ++i) qx[i] = Vec8<QT>::load(qp + (i >> 2) * 64 + (i & 3) * 8);
     if constexpr (RM == 1) {
-      // height/width pairs (global pair index cs * 32 + 16 hh + m >= 22) turned by the query's
-      // own position, in fp32 from the values above, then rounded to bf16 (the roped bf16
-      // query); temporal pairs stay as loaded and bound the scale by their norms.  Every product
-      // and sum rounds on its own (no contraction), so the fp8 codes are a fixed function of the
-      // inputs that a CPU restatement reproduces exactly.
-#pragma clang fp contract(off)
-      const int qr = qlive ? qrow : a.Lq - 1;
-      qfi = qr / a.T;
-      const int tt = qr - qfi * a.T, hq = tt / a.gw, wq = tt - hq * a.gw;
-      // every lane loads an in-bounds table entry and selects (no lane-divergent branches)
+      qfi = qrc / a.T;
+      const int tt = qrc - qfi * a.T, hq = tt / a.gw, wq = tt - hq * a.gw;
 #pragma unroll
       for (int cs = 0; cs < 2; ++cs)
 #pragma unroll
-        for (int m = 0; m < 16; ++m) {
+        for (int m = cs == 0 ? kRopeT - 16 : 0; m < 16; ++m) {
           const int pr = cs * 32 + hh * 16 + m;
-          const bool temporal = pr < kRopeT;
-          float& u = qv[cs * 32 + 2 * m];
-          float& v = qv[cs * 32 + 2 * m + 1];
           const int idx = pr < kRopeT + kRopeHW ? hq * kRopeHW + max(pr - kRopeT, 0)
                                                 : (a.gh + wq) * kRopeHW + (pr - kRopeT - kRopeHW);
-          const float2 cn = *reinterpret_cast<const float2*>(a.rope_hw + 2 * idx);
-          const float u2 = (float)(bf16)(u * cn.x - v * cn.y), v2 = (float)(bf16)(u * cn.y + v * cn.x);
-          const float bound = temporal ? __builtin_sqrtf(u * u + v * v)
-                                       : fmaxf(__builtin_fabsf(u2), __builtin_fabsf(v2));
-          amax = fmaxf(amax, bound);
-          u = temporal ? u : u2;
-          v = temporal ? v : v2;
+          qhw[cs][m] = *reinterpret_cast<const f32x2_u*>(a.rope_hw + 2 * idx);
         }
-      // slice 0 (channels 32 hh .. +31) to this wave's LDS rows: chunk c of lane L at c KB + 16 L
-      char* qs = lds + fp8_lds_bytes(NW) + w * kFp8QRows + lane * 16;
+    }
+  }
+  auto form_q = [&]() __attribute__((always_inline)) {
+    // the row in bf16 throughout (bf16 inputs, or the norm's / RoPE's bf16 outputs): chunk i holds
+    // channels (i >> 2) * 64 + 32 hh + 8 (i & 3) .. +7
+    Vec8<bf16> qb[8];
+    if (a.q_rms) {  // normalised Q in bf16, as the reference's norm_q output
+      const float qn = a.q_rms[(int64_t)b * a.q_rms_sb + qrc];
 #pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        bf16x8 t;
+      for (int i = 0; i < 8; ++i) {
+        const Vec8<float> wk = Vec8<float>::load(qw + (i >> 2) * 64 + (i & 3) * 8);
 #pragma unroll
-        for (int e = 0; e < 8; ++e) t[e] = (bf16)qv[8 * c + e];
-        *reinterpret_cast<bf16x8*>(qs + c * 1024) = t;
+        for (int j = 0; j < 8; ++j) qb[i].set(j, (bf16)((float)qx[i].get(j) * qn * wk.get(j)));
       }
     } else {
 #pragma unroll
-      for (int j = 0; j < 64; ++j) amax = fmaxf(amax, __builtin_fabsf(qv[j]));
+      for (int i = 0; i < 8; ++i)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) qb[i].set(j, (bf16)qx[i].get(j));
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) qb[i] = qlive ? qb[i] : Vec8<bf16>::zero();
+    float amax = 0.f;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      if constexpr (RM == 1) {
+        // height/width pairs (global pair index cs * 32 + 16 hh + m >= 22) turned by the query's
+        // own position, in fp32 from the values above, then rounded to bf16 (the roped bf16
+        // query); temporal pairs stay as loaded and bound the scale by their norms.  Every product
+        // and sum rounds on its own (no contraction), so the fp8 codes are a fixed function of the
+        // inputs that a CPU restatement reproduces exactly.
+#pragma clang fp contract(off)
+        const int cs = i >> 2;
+#pragma unroll
+        for (int mm = 0; mm < 4; ++mm) {
+          const int m = 4 * (i & 3) + mm;
+          const float u = (float)qb[i].get(2 * mm), v = (float)qb[i].get(2 * mm + 1);
+          const float norm = __builtin_sqrtf(u * u + v * v);
+          if (cs == 0 && m < kRopeT - 16) {  // temporal in both halves of the wave
+            amax = fmaxf(amax, norm);
+            continue;
+          }
+          const bool temporal = cs * 32 + hh * 16 + m < kRopeT;
+          const float cr = qhw[cs][m][0], sr = qhw[cs][m][1];
+          const bf16 u2 = (bf16)(u * cr - v * sr), v2 = (bf16)(u * sr + v * cr);
+          const float bound =
+              temporal ? norm : fmaxf(__builtin_fabsf((float)u2), __builtin_fabsf((float)v2));
+          amax = fmaxf(amax, bound);
+          qb[i].set(2 * mm, temporal ? (bf16)u : u2);
+          qb[i].set(2 * mm + 1, temporal ? (bf16)v : v2);
+        }
+      } else {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) amax = fmaxf(amax, __builtin_fabsf((float)qb[i].get(j)));
+      }
+    }
+    if constexpr (RM == 1) {
+      // slice 0 (channels 32 hh .. +31) to this wave's LDS rows: chunk c of lane L at c KB + 16 L
+      char* qs = lds + fp8_lds_bytes(NW) + w * kFp8QRows + lane * 16;
+#pragma unroll
+      for (int c = 0; c < 4; ++c) *reinterpret_cast<bf16x8*>(qs + c * 1024) = qb[c].to_bf16();
     }
     amax = pair_max(amax);
     const float inv = amax > 0.f ? 448.0f / amax : 0.f;
     q_scale = amax / 448.0f;
     q_inv = inv;
-    auto cl = [&](float x) { return fminf(fmaxf(x * inv, -448.f), 448.f); };
+    auto cl = [&](bf16 x) { return fminf(fmaxf((float)x * inv, -448.f), 448.f); };
 #pragma unroll
-    for (int cs = 0; cs < 2; ++cs)
+    for (int i = 0; i < 8; ++i)
 #pragma unroll
-      for (int d = 0; d < 8; ++d) {
-        const float* t = qv + cs * 32 + 4 * d;
-        q8[cs][d] = pack_fp8x4(cl(t[0]), cl(t[1]), cl(t[2]), cl(t[3]));
-      }
-  }
+      for (int d = 0; d < 2; ++d)
+        q8[i >> 2][2 * (i & 3) + d] =
+            pack_fp8x4(cl(qb[i].get(4 * d)), cl(qb[i].get(4 * d + 1)), cl(qb[i].get(4 * d + 2)),
+                       cl(qb[i].get(4 * d + 3)));
+  };
 
   const int n_keys = (int)a.n_keys;
   int lim_lane = n_keys, lim_lo = n_keys, lim_hi = n_keys;
@@ -1537,7 +1696,7 @@ void attn_fp8_kernel(AttnArgs a) {
   auto kb_lds = [&](int i) { return lds + (i & (kRing - 1)) * kBuf; };
   auto vb_lds = [&](int i) { return lds + (kRing + (i & (kRing - 1))) * kBuf; };
 
-  // RM = 1: the temporal angles of the q-tile's query frames qf_lo .. (at most kFp8TabFrames,
+  // RM = 1: the temporal angles of the q-tile's query frames qf_lo .. (at most kTabFrames,
   // checked by the host) against key frame j -> the table slot of the tile x that opens frame j
   // (slot x mod kRing, written with K(x) and read before QK(x), so it lives like K(x)'s buffer).
   // Lane i moves 16 bytes: pairs 2 (i % 11) .. +1 of query frame qf_lo + i / 11; lanes past the
@@ -1550,7 +1709,7 @@ void attn_fp8_kernel(AttnArgs a) {
       const int f = lane / 11, pp = lane - 11 * f;
       Stage64<1> st;
       st.goff[0] = (uint32_t)((((qf_lo + (f < count ? f : 0)) * a.n_frames + j) * kRopeT + 2 * pp) * 8);
-      st.loff[0] = (x & (kRing - 1)) * kFp8TabSlot;
+      st.loff[0] = (x & (kRing - 1)) * kTabSlot;
       st(reinterpret_cast<const uint8_t*>(a.rope_t), tab_lds);
     }
   };
@@ -1563,12 +1722,12 @@ void attn_fp8_kernel(AttnArgs a) {
     if constexpr (RM == 1) {
 #pragma clang fp contract(off)
       // pairs 16 hh .. +15 of the row's query frame (128 B from a 32-aligned offset inside the
-      // slot: (qfi - qf_lo) * 176 + 128 hh + 128 <= 4 * 176 + 256 < kFp8TabSlot), 4 pairs per
+      // slot: (qfi - qf_lo) * 176 + 128 hh + 128 <= 4 * 176 + 256 < kTabSlot), 4 pairs per
       // chunk c read by an asm block: the compiler's own LDS reads of a DMA-written buffer would
       // first wait for every DMA in flight (the next tiles' K and V), which the barrier after the
       // slot's DMA already covers
       const uint32_t tab = (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) char*)(
-          tab_lds + (x & (kRing - 1)) * kFp8TabSlot + (qfi - qf_lo) * (8 * kRopeT) + hh * 128);
+          tab_lds + (x & (kRing - 1)) * kTabSlot + (qfi - qf_lo) * (8 * kRopeT) + hh * 128);
       const char* qs = lds + fp8_lds_bytes(NW) + w * kFp8QRows + lane * 16;
       auto cl = [&](float v) { return fminf(fmaxf(v * q_inv, -448.f), 448.f); };
 #pragma unroll
@@ -1598,11 +1757,16 @@ void attn_fp8_kernel(AttnArgs a) {
     }
   };
 
+  // the window's largest V scale: the lanes load 64 frames' scales at once (a loop over the frames
+  // waits out a slot load and a scale load per frame, one after the other; H24 x 880 queries over
+  // 21 x 880 fp8 keys with RoPE: 258 -> 197 us a layer pass with the loads above)
   float sv_max = 0.f;
-  for (int j = 0; j < a.n_frames; ++j)
-    sv_max = fmaxf(sv_max, a.vscale[(int64_t)a.slots[j] * a.B * a.H + sc_bh]);
+  for (int j0 = 0; j0 < a.n_frames; j0 += 64)
+    sv_max = fmaxf(sv_max, a.vscale[(int64_t)a.slots[min(j0 + lane, a.n_frames - 1)] * a.B * a.H + sc_bh]);
+#pragma unroll
+  for (int d = 32; d > 0; d >>= 1) sv_max = fmaxf(sv_max, __shfl_xor(sv_max, d, 64));
+  sv_max = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(sv_max)));
   const float G = sv_max > 0.f ? 28.0f / sv_max : 1.0f;
-  const float c2q = a.scale_log2 * q_scale;
   const int lane16 = lane * 16;
 
   f32x16 oacc[4];
@@ -1654,6 +1818,7 @@ void attn_fp8_kernel(AttnArgs a) {
         }
       }
     }
+    form_q();
 #pragma unroll
     for (int r = 0; r < 8 / NW; ++r)
       *reinterpret_cast<u32x4*>(vb_lds(-1) + (tid + NW * 64 * r) * 16) = u32x4{0u, 0u, 0u, 0u};
@@ -1671,6 +1836,7 @@ void attn_fp8_kernel(AttnArgs a) {
   kw.start(a, kbh, tb + kL + 1);
   vw.start(a, kbh, tb + kL - 1);
   mw.start(a, kbh, tb + 1);
+  const float c2q = a.scale_log2 * q_scale;
   // Per key frame: the softmax multiplier (K scale folded in) and the log and reciprocal of the
   // P scale, for the frame of the tile whose softmax runs next.
   float mult = 0.f, log_pv = 0.f, inv_pv = 1.0f;
@@ -1816,6 +1982,7 @@ void attn_fp8_kernel(AttnArgs a) {
   };
   int tau = 0;
   for (; tau + 1 < ntau; tau += 2) {
+
     step(tau, 0, sA, sB, pA, pB);
     step(tau + 1, 1, sB, sA, pB, pA);
   }
@@ -1888,65 +2055,88 @@ void attn_fp8_kernel(AttnArgs a) {
 constexpr int kSplitBQ = 256;     // queries per q-tile of the split (8-wave) kernel
 constexpr int kMaxSplitWg = 1024;  // split grids have at most this many workgroups
 constexpr int kCombineRows = 4;    // rows per lane of attn_combine_kernel
+constexpr int kCombineRecs = 4;    // records it reads at a time
 constexpr int kCombineWgs = kSplitBQ / (8 * kCombineRows);  // its workgroups per q-tile
 
 template <typename QT>
 __global__ __launch_bounds__(256) void attn_combine_kernel(AttnArgs a) {
-  __shared__ int64_t recs[kMaxSplitWg];
-  __shared__ int n_rec;
   const int nt = a.nt;
   const int qg = blockIdx.x / kCombineWgs, rg = blockIdx.x % kCombineWgs;
-  const int64_t x0 = (int64_t)qg * nt, x1 = x0 + nt - 1;
-  auto lo = [&](int i) { return (int64_t)i * a.units / a.n_wg; };
-  auto owner = [&](int64_t x) {  // the workgroup whose range holds unit x
-    int i = (int)(x * a.n_wg / a.units);
-    while (i + 1 < a.n_wg && lo(i + 1) <= x) ++i;
-    while (i > 0 && lo(i) > x) --i;
+  const int x0 = qg * nt, x1 = x0 + nt - 1;
+  auto owner = [&](int x) {  // the workgroup whose (non-empty) share holds unit x
+    int i = min((int)((float)x / ((float)a.share_base + (float)a.share_rem / (float)a.n_wg)), a.n_wg - 1);
+    while (i + 1 < a.n_wg && share_begin(a, i + 1) <= x) ++i;
+    while (i > 0 && share_begin(a, i) > x) --i;
     return i;
   };
   const int i0 = owner(x0), i1 = owner(x1);
   if (i0 == i1) return;  // uniform: one workgroup covered the q-tile and wrote it
-  if (threadIdx.x == 0) {  // the records of this q-tile, once
-    int m = 0;
-    for (int i = i0; i <= i1; ++i)
-      if (lo(i) < lo(i + 1)) recs[m++] = 2 * (int64_t)i + (i == i0 && lo(i) < x0 ? 1 : 0);
-    n_rec = m;
-  }
-  __syncthreads();
-  const int nr = n_rec;
+  // its records: one per workgroup i0 .. i1, the last segment of i0's share when that share starts
+  // in an earlier q-tile
+  const int nr = i1 - i0 + 1;
+  const int first = 2 * i0 + (share_begin(a, i0) < x0 ? 1 : 0);
+  auto rec = [&](int p) { return (int64_t)(p == 0 ? first : 2 * (i0 + p)); };
+  // shares can only be empty (and their records unwritten) when there are fewer units than shares
+  auto live = [&](int p) {
+    return p < nr && (a.share_base > 0 || share_begin(a, i0 + p) < share_begin(a, i0 + p + 1));
+  };
   const int qt = (qg + a.qt_base) % a.n_qtiles, bh = (qg + a.qt_base) / a.n_qtiles;
   const int h = bh % a.H, b = bh / a.H;
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int c = (lane & 31) * 4;
   const int r0 = rg * (8 * kCombineRows) + 2 * w + (lane >> 5);  // rows r0 + 8 j
-  // rows past Lq read records in bounds (every record holds kSplitBQ rows) and store nothing
-  float M[kCombineRows];
-#pragma unroll
-  for (int j = 0; j < kCombineRows; ++j) M[j] = -INFINITY;
-  for (int p = 0; p < nr; ++p) {
-#pragma unroll
-    for (int j = 0; j < kCombineRows; ++j)
-      M[j] = fmaxf(M[j], a.part_ml[(recs[p] * kSplitBQ + r0 + 8 * j) * 2]);
-  }
-  float L[kCombineRows], o[kCombineRows][4];
+  // rows past Lq read records in bounds (every record holds kSplitBQ rows) and store nothing.
+  // Records are read kCombineRecs at a time, O and (max, sum) together (past the last, that one
+  // again with weight 0); up to that many (the usual case: a q-tile in 2 to 4 shares) are read once,
+  // before their common max is known, so a lane waits out one memory latency, not one per record.
+  float M[kCombineRows], L[kCombineRows], o[kCombineRows][4];
 #pragma unroll
   for (int j = 0; j < kCombineRows; ++j) {
+    M[j] = -INFINITY;
     L[j] = 0.f;
 #pragma unroll
     for (int e = 0; e < 4; ++e) o[j][e] = 0.f;
   }
-  for (int p = 0; p < nr; ++p) {
+  const bool once = nr <= kCombineRecs;
+  if (!once) {
+    for (int p0 = 0; p0 < nr; p0 += kCombineRecs) {
 #pragma unroll
-    for (int j = 0; j < kCombineRows; ++j) {
-      const int64_t row = recs[p] * kSplitBQ + r0 + 8 * j;
-      const float2 ml = *reinterpret_cast<const float2*>(a.part_ml + row * 2);
-      if (ml.x == -INFINITY) continue;
-      const float wgt = __builtin_amdgcn_exp2f(ml.x - M[j]);
-      const f32x4 v = *reinterpret_cast<const f32x4*>(a.part_o + row * kHeadDim + c);
-      L[j] = fmaf(wgt, ml.y, L[j]);
+      for (int k = 0; k < kCombineRecs; ++k)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) o[j][e] = fmaf(wgt, v[e], o[j][e]);
+        for (int j = 0; j < kCombineRows; ++j)
+        {
+          const float m = a.part_ml[(rec(min(p0 + k, nr - 1)) * kSplitBQ + r0 + 8 * j) * 2];
+          M[j] = fmaxf(M[j], live(p0 + k) ? m : -INFINITY);
+        }
     }
+  }
+  for (int p0 = 0; p0 < nr; p0 += kCombineRecs) {
+    float2 ml[kCombineRecs][kCombineRows];
+    f32x4 v[kCombineRecs][kCombineRows];
+#pragma unroll
+    for (int k = 0; k < kCombineRecs; ++k)
+#pragma unroll
+      for (int j = 0; j < kCombineRows; ++j) {
+        const int64_t row = rec(min(p0 + k, nr - 1)) * kSplitBQ + r0 + 8 * j;
+        ml[k][j] = *reinterpret_cast<const float2*>(a.part_ml + row * 2);
+        v[k][j] = *reinterpret_cast<const f32x4*>(a.part_o + row * kHeadDim + c);
+      }
+    if (once) {
+#pragma unroll
+      for (int j = 0; j < kCombineRows; ++j)
+#pragma unroll
+        for (int k = 0; k < kCombineRecs; ++k) M[j] = fmaxf(M[j], live(k) ? ml[k][j].x : -INFINITY);
+    }
+#pragma unroll
+    for (int k = 0; k < kCombineRecs; ++k)
+#pragma unroll
+      for (int j = 0; j < kCombineRows; ++j) {
+        const bool use = live(p0 + k) && ml[k][j].x != -INFINITY;
+        const float wgt = use ? __builtin_amdgcn_exp2f(ml[k][j].x - M[j]) : 0.f;
+        L[j] = use ? fmaf(wgt, ml[k][j].y, L[j]) : L[j];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[j][e] = use ? fmaf(wgt, v[k][j][e], o[j][e]) : o[j][e];
+      }
   }
 #pragma unroll
   for (int j = 0; j < kCombineRows; ++j) {
@@ -1998,37 +2188,37 @@ static void launch(const AttnArgs& a, int q_dtype, int pool_dtype, int rm, hipSt
     if constexpr (NW == 8) {
       if (a.split) {
         if (a.packed) {
-          if (qh) hipLaunchKernelGGL((attn_kernel<NW, f16, f16, 0, true, true>), grid, block, attn_lds_bytes(NW, 0, 2, true, true), s, a);
-          else hipLaunchKernelGGL((attn_kernel<NW, float, f16, 0, true, true>), grid, block, attn_lds_bytes(NW, 0, 2, true, true), s, a);
+          if (qh) hipLaunchKernelGGL((attn_kernel<NW, f16, f16, 0, true, true>), grid, block, attn_lds_bytes(NW, 0, 2), s, a);
+          else hipLaunchKernelGGL((attn_kernel<NW, float, f16, 0, true, true>), grid, block, attn_lds_bytes(NW, 0, 2), s, a);
         } else {
-          if (qh) hipLaunchKernelGGL((attn_kernel<NW, f16, f16, 0, true>), grid, block, attn_lds_bytes(NW, 0, 2, true, false), s, a);
-          else hipLaunchKernelGGL((attn_kernel<NW, float, f16, 0, true>), grid, block, attn_lds_bytes(NW, 0, 2, true, false), s, a);
+          if (qh) hipLaunchKernelGGL((attn_kernel<NW, f16, f16, 0, true>), grid, block, attn_lds_bytes(NW, 0, 2), s, a);
+          else hipLaunchKernelGGL((attn_kernel<NW, float, f16, 0, true>), grid, block, attn_lds_bytes(NW, 0, 2), s, a);
         }
         return;
       }
     }
     if (a.packed) {
-      if (qh) hipLaunchKernelGGL((attn_kernel<NW, f16, f16, 0, false, true>), grid, block, attn_lds_bytes(NW, 0, 2, false, true), s, a);
-      else hipLaunchKernelGGL((attn_kernel<NW, float, f16, 0, false, true>), grid, block, attn_lds_bytes(NW, 0, 2, false, true), s, a);
+      if (qh) hipLaunchKernelGGL((attn_kernel<NW, f16, f16, 0, false, true>), grid, block, attn_lds_bytes(NW, 0, 2), s, a);
+      else hipLaunchKernelGGL((attn_kernel<NW, float, f16, 0, false, true>), grid, block, attn_lds_bytes(NW, 0, 2), s, a);
     } else {
-      if (qh) hipLaunchKernelGGL((attn_kernel<NW, f16, f16, 0>), grid, block, attn_lds_bytes(NW, 0, 2, false, false), s, a);
-      else hipLaunchKernelGGL((attn_kernel<NW, float, f16, 0>), grid, block, attn_lds_bytes(NW, 0, 2, false, false), s, a);
+      if (qh) hipLaunchKernelGGL((attn_kernel<NW, f16, f16, 0>), grid, block, attn_lds_bytes(NW, 0, 2), s, a);
+      else hipLaunchKernelGGL((attn_kernel<NW, float, f16, 0>), grid, block, attn_lds_bytes(NW, 0, 2), s, a);
     }
     return;
   }
   // fp8 pools with RoPE on load: the fp8-MFMA kernel (query temporal pairs rebuilt per key
-  // frame) when a q-tile spans at most kFp8TabFrames query frames (frames of >= 64 tokens);
+  // frame) when a q-tile spans at most kTabFrames query frames (frames of >= 64 tokens);
   // shorter frames and fused PRoPE take the bf16 kernel staging decoded tiles (PRoPE's
   // per-key-frame W is unbounded, so the query cannot keep one fp8 scale).  bf16 queries
   // (checked by the caller).
   if (pool_dtype == SKV_FP8_E4M3 && rm == 1 && a.T < kTile) {
     if constexpr (NW == 8) {
       if (a.split) {
-        hipLaunchKernelGGL((attn_kernel<NW, bf16, fp8e4, 1, true>), grid, block, attn_lds_bytes(NW, 1, 1, true, false), s, a);
+        hipLaunchKernelGGL((attn_kernel<NW, bf16, fp8e4, 1, true>), grid, block, attn_lds_bytes(NW, 1, 1), s, a);
         return;
       }
     }
-    hipLaunchKernelGGL((attn_kernel<NW, bf16, fp8e4, 1>), grid, block, attn_lds_bytes(NW, 1, 1, false, false), s, a);
+    hipLaunchKernelGGL((attn_kernel<NW, bf16, fp8e4, 1>), grid, block, attn_lds_bytes(NW, 1, 1), s, a);
     return;
   }
   if (pool_dtype == SKV_FP8_E4M3 && rm == 1) {
@@ -2044,11 +2234,11 @@ static void launch(const AttnArgs& a, int q_dtype, int pool_dtype, int rm, hipSt
   if (pool_dtype == SKV_FP8_E4M3 && rm == 2) {  // bf16 queries (checked by the caller)
     if constexpr (NW == 8) {
       if (a.split) {
-        hipLaunchKernelGGL((attn_kernel<NW, bf16, fp8e4, 2, true>), grid, block, attn_lds_bytes(NW, 2, 1, true, false), s, a);
+        hipLaunchKernelGGL((attn_kernel<NW, bf16, fp8e4, 2, true>), grid, block, attn_lds_bytes(NW, 2, 1), s, a);
         return;
       }
     }
-    hipLaunchKernelGGL((attn_kernel<NW, bf16, fp8e4, 2>), grid, block, attn_lds_bytes(NW, 2, 1, false, false), s, a);
+    hipLaunchKernelGGL((attn_kernel<NW, bf16, fp8e4, 2>), grid, block, attn_lds_bytes(NW, 2, 1), s, a);
     return;
   }
   if (pool_dtype == SKV_FP8_E4M3) {
@@ -2071,51 +2261,61 @@ static void launch(const AttnArgs& a, int q_dtype, int pool_dtype, int rm, hipSt
     if (a.split) {  // bf16 or fp32 pools, no mask (checked by the caller)
       const bool qb = q_dtype == SKV_BF16;
       if (rm == 2) {
-        if (qb) hipLaunchKernelGGL((attn_kernel<NW, bf16, bf16, 2, true>), grid, block, attn_lds_bytes(NW, 2, 2, true, false), s, a);
-        else hipLaunchKernelGGL((attn_kernel<NW, float, bf16, 2, true>), grid, block, attn_lds_bytes(NW, 2, 2, true, false), s, a);
+        if (qb) hipLaunchKernelGGL((attn_kernel<NW, bf16, bf16, 2, true>), grid, block, attn_lds_bytes(NW, 2, 2), s, a);
+        else hipLaunchKernelGGL((attn_kernel<NW, float, bf16, 2, true>), grid, block, attn_lds_bytes(NW, 2, 2), s, a);
+      } else if (rm == 1 && !a.rope_lds) {
+        if (qb) hipLaunchKernelGGL((attn_kernel<NW, bf16, bf16, 3, true>), grid, block, attn_lds_bytes(NW, 3, 2), s, a);
+        else hipLaunchKernelGGL((attn_kernel<NW, float, bf16, 3, true>), grid, block, attn_lds_bytes(NW, 3, 2), s, a);
       } else if (rm == 1) {
-        if (qb) hipLaunchKernelGGL((attn_kernel<NW, bf16, bf16, 1, true>), grid, block, attn_lds_bytes(NW, 1, 2, true, false), s, a);
-        else hipLaunchKernelGGL((attn_kernel<NW, float, bf16, 1, true>), grid, block, attn_lds_bytes(NW, 1, 2, true, false), s, a);
+        if (qb) hipLaunchKernelGGL((attn_kernel<NW, bf16, bf16, 1, true>), grid, block, attn_lds_bytes(NW, 1, 2), s, a);
+        else hipLaunchKernelGGL((attn_kernel<NW, float, bf16, 1, true>), grid, block, attn_lds_bytes(NW, 1, 2), s, a);
       } else if (pool_dtype == SKV_BF16 && a.packed) {
-        if (qb) hipLaunchKernelGGL((attn_kernel<NW, bf16, bf16, 0, true, true>), grid, block, attn_lds_bytes(NW, 0, 2, true, true), s, a);
-        else hipLaunchKernelGGL((attn_kernel<NW, float, bf16, 0, true, true>), grid, block, attn_lds_bytes(NW, 0, 2, true, true), s, a);
+        if (qb) hipLaunchKernelGGL((attn_kernel<NW, bf16, bf16, 0, true, true>), grid, block, attn_lds_bytes(NW, 0, 2), s, a);
+        else hipLaunchKernelGGL((attn_kernel<NW, float, bf16, 0, true, true>), grid, block, attn_lds_bytes(NW, 0, 2), s, a);
       } else if (pool_dtype == SKV_BF16) {
-        if (qb) hipLaunchKernelGGL((attn_kernel<NW, bf16, bf16, 0, true>), grid, block, attn_lds_bytes(NW, 0, 2, true, false), s, a);
-        else hipLaunchKernelGGL((attn_kernel<NW, float, bf16, 0, true>), grid, block, attn_lds_bytes(NW, 0, 2, true, false), s, a);
+        if (qb) hipLaunchKernelGGL((attn_kernel<NW, bf16, bf16, 0, true>), grid, block, attn_lds_bytes(NW, 0, 2), s, a);
+        else hipLaunchKernelGGL((attn_kernel<NW, float, bf16, 0, true>), grid, block, attn_lds_bytes(NW, 0, 2), s, a);
       } else {
-        if (qb) hipLaunchKernelGGL((attn_kernel<NW, bf16, float, 0, true>), grid, block, attn_lds_bytes(NW, 0, 4, true, false), s, a);
-        else hipLaunchKernelGGL((attn_kernel<NW, float, float, 0, true>), grid, block, attn_lds_bytes(NW, 0, 4, true, false), s, a);
+        if (qb) hipLaunchKernelGGL((attn_kernel<NW, bf16, float, 0, true>), grid, block, attn_lds_bytes(NW, 0, 4), s, a);
+        else hipLaunchKernelGGL((attn_kernel<NW, float, float, 0, true>), grid, block, attn_lds_bytes(NW, 0, 4), s, a);
       }
       return;
     }
   }
   if (rm == 2) {  // bf16 pools, frame_tokens >= 64 (checked by the caller)
     if (q_dtype == SKV_BF16)
-      hipLaunchKernelGGL((attn_kernel<NW, bf16, bf16, 2>), grid, block, attn_lds_bytes(NW, 2, 2, false, false), s, a);
+      hipLaunchKernelGGL((attn_kernel<NW, bf16, bf16, 2>), grid, block, attn_lds_bytes(NW, 2, 2), s, a);
     else
-      hipLaunchKernelGGL((attn_kernel<NW, float, bf16, 2>), grid, block, attn_lds_bytes(NW, 2, 2, false, false), s, a);
+      hipLaunchKernelGGL((attn_kernel<NW, float, bf16, 2>), grid, block, attn_lds_bytes(NW, 2, 2), s, a);
     return;
   }
-  if (rm == 1) {  // bf16 pools only (checked by the caller)
+  if (rm == 1 && !a.rope_lds) {  // bf16 pools only (checked by the caller)
     if (q_dtype == SKV_BF16)
-      hipLaunchKernelGGL((attn_kernel<NW, bf16, bf16, 1>), grid, block, attn_lds_bytes(NW, 1, 2, false, false), s, a);
+      hipLaunchKernelGGL((attn_kernel<NW, bf16, bf16, 3>), grid, block, attn_lds_bytes(NW, 3, 2), s, a);
     else
-      hipLaunchKernelGGL((attn_kernel<NW, float, bf16, 1>), grid, block, attn_lds_bytes(NW, 1, 2, false, false), s, a);
+      hipLaunchKernelGGL((attn_kernel<NW, float, bf16, 3>), grid, block, attn_lds_bytes(NW, 3, 2), s, a);
+    return;
+  }
+  if (rm == 1) {
+    if (q_dtype == SKV_BF16)
+      hipLaunchKernelGGL((attn_kernel<NW, bf16, bf16, 1>), grid, block, attn_lds_bytes(NW, 1, 2), s, a);
+    else
+      hipLaunchKernelGGL((attn_kernel<NW, float, bf16, 1>), grid, block, attn_lds_bytes(NW, 1, 2), s, a);
     return;
   }
   if (pool_dtype == SKV_BF16 && a.packed) {
     if (q_dtype == SKV_BF16)
-      hipLaunchKernelGGL((attn_kernel<NW, bf16, bf16, 0, false, true>), grid, block, attn_lds_bytes(NW, 0, 2, false, true), s, a);
+      hipLaunchKernelGGL((attn_kernel<NW, bf16, bf16, 0, false, true>), grid, block, attn_lds_bytes(NW, 0, 2), s, a);
     else
-      hipLaunchKernelGGL((attn_kernel<NW, float, bf16, 0, false, true>), grid, block, attn_lds_bytes(NW, 0, 2, false, true), s, a);
+      hipLaunchKernelGGL((attn_kernel<NW, float, bf16, 0, false, true>), grid, block, attn_lds_bytes(NW, 0, 2), s, a);
   } else if (q_dtype == SKV_BF16 && pool_dtype == SKV_BF16)
-    hipLaunchKernelGGL((attn_kernel<NW, bf16, bf16, 0>), grid, block, attn_lds_bytes(NW, 0, 2, false, false), s, a);
+    hipLaunchKernelGGL((attn_kernel<NW, bf16, bf16, 0>), grid, block, attn_lds_bytes(NW, 0, 2), s, a);
   else if (q_dtype == SKV_BF16 && pool_dtype == SKV_F32)
-    hipLaunchKernelGGL((attn_kernel<NW, bf16, float, 0>), grid, block, attn_lds_bytes(NW, 0, 4, false, false), s, a);
+    hipLaunchKernelGGL((attn_kernel<NW, bf16, float, 0>), grid, block, attn_lds_bytes(NW, 0, 4), s, a);
   else if (q_dtype == SKV_F32 && pool_dtype == SKV_BF16)
-    hipLaunchKernelGGL((attn_kernel<NW, float, bf16, 0>), grid, block, attn_lds_bytes(NW, 0, 2, false, false), s, a);
+    hipLaunchKernelGGL((attn_kernel<NW, float, bf16, 0>), grid, block, attn_lds_bytes(NW, 0, 2), s, a);
   else
-    hipLaunchKernelGGL((attn_kernel<NW, float, float, 0>), grid, block, attn_lds_bytes(NW, 0, 4, false, false), s, a);
+    hipLaunchKernelGGL((attn_kernel<NW, float, float, 0>), grid, block, attn_lds_bytes(NW, 0, 4), s, a);
 }
 
 static int attention_impl(const void* q, int q_dtype, int64_t q_sb, int64_t q_st,
@@ -2286,6 +2486,9 @@ static int attention_impl(const void* q, int q_dtype, int64_t q_sb, int64_t q_st
   a.q_rms = q_inv_rms;
   a.q_rms_sb = q_rms_sb;
   a.q_w = q_norm_weight;
+  // shorter frames would put more than kTabFrames query frames into a q-tile; the offsets are 32-bit
+  a.rope_lds = rope && frame_tokens >= kTile &&
+               (int64_t)n_qframes * n_frames * 8 * kRopeT < ((int64_t)1 << 31);
   a.gh = grid_h;
   a.gw = grid_w;
   a.n_qframes = n_qframes;
@@ -2362,7 +2565,7 @@ static int attention_impl(const void* q, int q_dtype, int64_t q_sb, int64_t q_st
   // H24 x 18480 keys, B 1 and 2), so 4-wave grids split at a smaller margin: the split also
   // moves them onto the 8-wave kernel (C3: 0.598 -> 0.571 ms, B 2: 1.246 -> 1.154 ms).
   a.split = 0;
-  a.units = 0;
+  a.share_base = a.share_rem = 0;
   a.qt_base = 0;
   a.part_o = a.part_ml = nullptr;
   int64_t split_bytes = 0;
@@ -2371,6 +2574,7 @@ static int attention_impl(const void* q, int q_dtype, int64_t q_sb, int64_t q_st
   const int64_t qt8 = (int64_t)((q_len + kSplitBQ - 1) / kSplitBQ) * heads * batch;
   const int64_t units8 = qt8 * nt;
   if (mask_mode == SKV_MASK_NONE && n_segments == 0 && nt >= 8 && units8 >= 4 * n_cu &&
+      units8 < ((int64_t)1 << 31) &&
       n_cu <= kMaxSplitWg) {
     auto t_tile = [&](int64_t busy) { return 1.0 + 0.62 * (double)busy / n_cu; };
     auto t_grid = [&](int64_t wg, int per_cu, double per_tile) {  // rounds of nt tiles
@@ -2410,7 +2614,8 @@ static int attention_impl(const void* q, int q_dtype, int64_t q_sb, int64_t q_st
       a.split = 1;
       a.n_qtiles = (int)(qt8 / ((int64_t)heads * batch));
       a.n_wg = n_cu;
-      a.units = units8;
+      a.share_base = (int)(units8 / n_cu);
+      a.share_rem = (int)(units8 % n_cu);
     } else {
       a.split = 2;  // launched below as an unsplit grid of the full rounds, then the tail
     }
@@ -2476,13 +2681,14 @@ static int attention_impl(const void* q, int q_dtype, int64_t q_sb, int64_t q_st
     AttnArgs t = a;
     t.split = 1;
     t.n_wg = n_cu;
-    t.units = (int64_t)n_tail * nt;
+    t.share_base = n_tail * nt / n_cu;
+    t.share_rem = n_tail * nt % n_cu;
     t.qt_base = (int)full_wg;
     launch<8>(t, q_dtype, pool_dtype, rm, s);
     combine(t, n_tail);
   } else if (a.n_seg > 0) {
     dim3 grid(a.n_wg), block(512);
-    const size_t lds = attn_lds_bytes(8, 0, 2, false, a.packed);
+    const size_t lds = attn_lds_bytes(8, 0, 2);
     if (a.packed) {
       if (q_dtype == SKV_BF16) hipLaunchKernelGGL((attn_kernel<8, bf16, bf16, 0, false, true, true>), grid, block, lds, s, a);
       else hipLaunchKernelGGL((attn_kernel<8, float, bf16, 0, false, true, true>), grid, block, lds, s, a);
