@@ -257,6 +257,15 @@ typedef struct skv_append_desc {
 int skv_append_ex(const skv_append_desc* desc, skv_stream_t stream);
 
 /*
+ * skv_append_round — a float32 chunk into bf16 pools, each value rounded once to bf16 (nearest
+ * even): the staging of dense float32 attention calls (attention.py:141-188 casts such inputs to
+ * bf16 before its kernel; the attention here multiplies float32 K/V in bf16 too).  No K norm, no
+ * RoPE / PRoPE copies; every other pool and source type is refused, as skv_append_ex refuses
+ * this one.
+ */
+int skv_append_round(const skv_append_desc* desc, skv_stream_t stream);
+
+/*
  * Workspace skv_append_ex would use for `desc` (0 when the launch needs none: bf16/f32 pools,
  * or an fp8 chunk with enough units to fill the chip); validates like skv_append_ex.  No
  * reference counterpart (the reference append, causal_model.py:2894-2914, is a slice copy).

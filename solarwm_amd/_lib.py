@@ -137,6 +137,7 @@ SIGNATURES: dict[str, tuple] = {
         [_vp, _i32, _i64, _i64, _i64, _i32, _i32, _i32, _i32, _f32, _vp, _vp],
     ),
     "skv_append_ex": (_i32, [ctypes.POINTER(AppendDesc), _vp]),
+    "skv_append_round": (_i32, [ctypes.POINTER(AppendDesc), _vp]),
     "skv_attention_ex": (_i32, [ctypes.POINTER(AttentionDesc), _vp]),
     "skv_attention_plan": (_i32, [ctypes.POINTER(AttentionDesc), ctypes.POINTER(LaunchPlan)]),
     "skv_attention_ex_noalloc": (_i32, [ctypes.POINTER(AttentionDesc), _vp]),

@@ -27,17 +27,10 @@ from .prope import CameraPass, commit_camera_cache, stage_camera_cache
 from .rope import positions as rope_positions
 
 
-def _pack_dense(k: torch.Tensor, v: torch.Tensor, pool_dtype: torch.dtype):
-    """Stage dense K/V [B, L, H, D] as a one-frame pool (V transposed) for the kernel, in this
-    stream's reused staging buffer (no allocation or zero-fill per call)."""
-    b, lk, h, _ = k.shape
-    kpool, vpool = kernels.staging_pools(1, b, h, lk, pool_dtype, k.device)
-    kernels.append_frames(k, v, kpool, vpool, [0], frame_tokens=lk)
-    return kpool, vpool
-
-
 def _dense_attention(q, k, v, softmax_scale, mask_mode=_lib.SKV_MASK_NONE, q_pos0=0, chunk=0):
-    kpool, vpool = _pack_dense(k, v, k.dtype)
+    # dense K/V as a one-frame pool (V transposed) in this stream's reused staging buffer (no
+    # allocation or zero-fill per call)
+    kpool, vpool = kernels.stage_frames(k, v, 1, k.shape[1])
     return kernels.attention_frames(
         q, kpool, vpool, [0], frame_tokens=k.shape[1], softmax_scale=softmax_scale,
         mask_mode=mask_mode, q_pos0=q_pos0, chunk_tokens=chunk,
@@ -78,7 +71,8 @@ def attention(
     # attention.py:69-87: inputs that are not half precision are cast to `dtype`, then q and k
     # to v's dtype, and the kernel computes in that dtype.  bf16 runs the bf16 MFMA kernel (fp32
     # inputs with dtype=bfloat16 are passed as fp32 and rounded to bf16 on load, the same
-    # rounding); fp16 runs the same kernel on fp16 pools with fp16 MFMAs.
+    # rounding; K and V are rounded once, when they are staged); fp16 runs the same kernel on fp16
+    # pools with fp16 MFMAs.
     half = (torch.float16, torch.bfloat16)
 
     def to_half(x):

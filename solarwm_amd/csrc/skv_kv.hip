@@ -240,6 +240,59 @@ __global__ __launch_bounds__(256) void append_kernel(AppendArgs a) {
   }
 }
 
+// Float32 chunk -> bf16 pool (skv_append_round), each value rounded once to nearest even: the same
+// split of a tile as append_kernel.  The dense attention calls stage float32 K/V through it: the
+// attention kernels multiply float32 inputs in bf16, so a float32 pool only made every q-tile
+// workgroup read twice the bytes and round them again, in registers, on the way to LDS.  H12, 1170
+// float32 queries over 8190 keys: 169 -> 118 us a call.  Memory bound (101 MB read, 50 MB written);
+// plain stores: the attention that follows reads the pool at once.
+__global__ __launch_bounds__(256) void append_round_kernel(AppendArgs a) {
+  int wg = blockIdx.x;
+  const int t = wg % a.ntiles;
+  wg /= a.ntiles;
+  const int h = wg % a.H;
+  wg /= a.H;
+  const int b = wg % a.B;
+  const int f = wg / a.B;
+  const int64_t slot = a.slots[f];
+  const int tid = threadIdx.x, tok0 = t * kTile;
+  const int64_t src_base = (int64_t)b * a.s_sb + (int64_t)h * a.s_sh +
+                           (int64_t)(a.src_frame0 + f) * a.T * a.s_st;
+  // every load before the first store; rows past T load the last row and are stored as zeros
+  Vec8<float> in[8];
+  u32x4 r16[8];
+  if (tid < 128) {
+    const float* ks = static_cast<const float*>(a.ksrc);
+    bf16* kp = static_cast<bf16*>(a.kpool) + slot * a.slot_stride +
+               ((int64_t)(b * a.H + h) * a.Tp + tok0) * kHeadDim;
+    const int col = (tid & 15) * 8, row0 = tid >> 4;
+#pragma unroll
+    for (int r = 0; r < 8; ++r)
+      in[r] = Vec8<float>::load_nt(ks + src_base + (int64_t)min(tok0 + row0 + 8 * r, a.T - 1) * a.s_st + col);
+#pragma unroll
+    for (int r = 0; r < 8; ++r) {
+      const int row = row0 + 8 * r;
+      r16[r] = tok0 + row < a.T ? __builtin_bit_cast(u32x4, in[r].to_bf16()) : u32x4{0u, 0u, 0u, 0u};
+      *reinterpret_cast<u32x4*>(kp + row * kHeadDim + col) = r16[r];
+    }
+    return;
+  }
+  const float* vs = static_cast<const float*>(a.vsrc);
+  bf16* vp = static_cast<bf16*>(a.vpool) + slot * a.slot_stride +
+             (int64_t)(b * a.H + h) * kHeadDim * a.Tp + tok0;
+  const int tb = (tid - 128) & 7, db = (tid - 128) >> 3;
+#pragma unroll
+  for (int r = 0; r < 8; ++r)
+    in[r] = Vec8<float>::load_nt(vs + src_base + (int64_t)min(tok0 + tb * 8 + r, a.T - 1) * a.s_st + db * 8);
+#pragma unroll
+  for (int r = 0; r < 8; ++r)
+    r16[r] = tok0 + tb * 8 + r < a.T ? __builtin_bit_cast(u32x4, in[r].to_bf16()) : u32x4{0u, 0u, 0u, 0u};
+  u32x4 out[8];
+  transpose8x8_b16(r16, out);
+#pragma unroll
+  for (int c = 0; c < 8; ++c) *reinterpret_cast<u32x4*>(vp + (int64_t)(db * 8 + c) * a.Tp + tb * 8) = out[c];
+}
+
 // fp8 append with the frame held on chip (bf16 sources, Tp <= 64 * kFp8OnChip): one
 // 1024-thread workgroup per (frame, batch, head, K|V); thread t owns chunk j = 16 B of row
 // 64 j + t / 16, channels (t % 16) * 8 .. +8.  Every chunk of the frame is loaded at once (one
@@ -1116,7 +1169,7 @@ static int append_impl(const void* k_new, const void* v_new, int src_dtype, int6
                        const float* k_inv_rms = nullptr, int64_t rms_sb = 0,
                        const float* k_norm_weight = nullptr, void* workspace = nullptr,
                        int64_t workspace_bytes = 0, int64_t* ws_query = nullptr,
-                       float* kr_scale = nullptr, float* vr_scale = nullptr) {
+                       float* kr_scale = nullptr, float* vr_scale = nullptr, bool round = false) {
   if (ws_query) *ws_query = 0;
   if (!k_new || !v_new || !k_pool || !v_pool || !dst_slots) {
     set_error("skv_append: null pointer argument");
@@ -1139,8 +1192,13 @@ static int append_impl(const void* k_new, const void* v_new, int src_dtype, int6
   }
   if (n_frames == 0) return SKV_OK;
   const bool fp8 = pool_dtype == SKV_FP8_E4M3;
-  if (!(src_dtype == SKV_BF16 || src_dtype == SKV_F32 || src_dtype == SKV_F16) ||
-      !(pool_dtype == src_dtype || (fp8 && src_dtype != SKV_F16))) {
+  if (round) {
+    if (src_dtype != SKV_F32 || pool_dtype != SKV_BF16 || kr_pool || vr_pool || kv_xform || k_inv_rms) {
+      set_error("skv_append_round: float32 chunks into bf16 pools only (no K norm, no copies)");
+      return SKV_E_UNSUPPORTED;
+    }
+  } else if (!(src_dtype == SKV_BF16 || src_dtype == SKV_F32 || src_dtype == SKV_F16) ||
+             !(pool_dtype == src_dtype || (fp8 && src_dtype != SKV_F16))) {
     set_error("skv_append: src_dtype=%d pool_dtype=%d unsupported (pool must equal src or be fp8)",
               src_dtype, pool_dtype);
     return SKV_E_UNSUPPORTED;
@@ -1313,7 +1371,9 @@ static int append_impl(const void* k_new, const void* v_new, int src_dtype, int6
     if (copy_units) return append_fp8_copies(a, src_dtype, copy_units, workspace, s);
   } else {
     dim3 grid(n_frames * batch * heads * a.ntiles);
-    if (src_dtype == SKV_BF16 || src_dtype == SKV_F16) {
+    if (round) {
+      hipLaunchKernelGGL(append_round_kernel, grid, dim3(256), 0, s, a);
+    } else if (src_dtype == SKV_BF16 || src_dtype == SKV_F16) {
       if (kv_xform)
         hipLaunchKernelGGL((append_kernel<bf16, 2>), grid, dim3(256), 0, s, a);
       else if (kr_pool)
@@ -1377,7 +1437,8 @@ extern "C" int skv_append_prope(const void* k_new, const void* v_new, int src_dt
                      stream);
 }
 
-static int append_desc(const skv_append_desc* d, skv_stream_t stream, int64_t* ws_query) {
+static int append_desc(const skv_append_desc* d, skv_stream_t stream, int64_t* ws_query,
+                       bool round = false) {
   clear_error();
   if (!d) {
     set_error("skv_append_ex: null descriptor");
@@ -1392,11 +1453,15 @@ static int append_desc(const skv_append_desc* d, skv_stream_t stream, int64_t* w
                      d->n_slots, d->dst_slots, d->n_frames, d->batch, d->heads, d->head_dim,
                      d->frame_tokens, d->kr_pool, d->rope_hw, d->grid_h, d->grid_w, d->vx_pool,
                      d->kv_xform, stream, d->k_inv_rms, d->k_rms_stride_b, d->k_norm_weight,
-                     d->workspace, d->workspace_bytes, ws_query, d->kr_scale, d->vx_scale);
+                     d->workspace, d->workspace_bytes, ws_query, d->kr_scale, d->vx_scale, round);
 }
 
 extern "C" int skv_append_ex(const skv_append_desc* d, skv_stream_t stream) {
   return append_desc(d, stream, nullptr);
+}
+
+extern "C" int skv_append_round(const skv_append_desc* d, skv_stream_t stream) {
+  return append_desc(d, stream, nullptr, true);
 }
 
 extern "C" int skv_append_workspace_size(const skv_append_desc* d, int64_t* bytes) {

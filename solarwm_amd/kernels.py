@@ -247,6 +247,7 @@ def prepare_append(
     use_workspace: bool = True,
     kr_scale: torch.Tensor | None = None,
     vr_scale: torch.Tensor | None = None,
+    entry: str = "skv_append_ex",
 ):
     """Validate an append once and return a zero-argument launcher that enqueues it on the stream
     current now (repeated launches skip the Python-side checks).
@@ -332,11 +333,11 @@ def prepare_append(
                    lib.skv_append_workspace_size(ctypes.byref(desc), ctypes.byref(need)))
         desc.workspace, desc.workspace_bytes, ws_tensor = workspace(kpool.device, need.value)
     args = (ctypes.byref(desc), _stream(kpool.device))
-    fn = lib.skv_append_ex
+    fn = getattr(lib, entry)
 
     def launch() -> None:
         t0 = _tic("append")
-        _lib.check("skv_append_ex", fn(*args))
+        _lib.check(entry, fn(*args))
         _toc("append", t0, moved)
 
     launch.bytes_moved = moved
@@ -377,6 +378,24 @@ def append_frames(
                    rope_hw=rope_hw, grid_hw=grid_hw, vr_pool=vr_pool, kv_xform=kv_xform,
                    k_norm=k_norm, use_workspace=use_workspace, kr_scale=kr_scale,
                    vr_scale=vr_scale)()
+
+
+def stage_frames(k: torch.Tensor, v: torch.Tensor, n_frames: int, frame_tokens: int,
+                 ) -> tuple[torch.Tensor, torch.Tensor]:
+    """Dense ``k`` / ``v`` [B, n_frames * frame_tokens, H, D] (bf16, f16 or float32) staged as frames
+    0.. of this stream's staging pools (:func:`staging_pools`) for an attention launch; returns the
+    pools.  float32 values are rounded to bf16, which is how the attention multiplies them: a bf16
+    pool halves what its workgroups read and needs no rounding on the way to LDS."""
+    b, _, h, _ = k.shape
+    if k.dtype != torch.float32:
+        kpool, vpool = staging_pools(n_frames, b, h, frame_tokens, k.dtype, k.device)
+        append_frames(k, v, kpool, vpool, list(range(n_frames)), frame_tokens=frame_tokens)
+        return kpool, vpool
+    kpool, vpool = staging_pools(n_frames, b, h, frame_tokens, torch.bfloat16, k.device)
+    launch = prepare_append(k, v, kpool, vpool, list(range(n_frames)), frame_tokens=frame_tokens,
+                            entry="skv_append_round")
+    launch()
+    return kpool, vpool
 
 
 def prepare_gather(
