@@ -197,6 +197,12 @@ typedef __attribute__((address_space(1))) void glb_void_t;
 // vector loads from caller tables that are only known to be float-aligned
 typedef float f32x2_u __attribute__((ext_vector_type(2), aligned(4)));
 typedef float f32x4_u __attribute__((ext_vector_type(4), aligned(4)));
+__device__ inline Vec8<float> load8_u(const float* p) {
+  Vec8<float> v;
+  v.a = *reinterpret_cast<const f32x4_u*>(p);
+  v.b = *reinterpret_cast<const f32x4_u*>(p + 4);
+  return v;
+}
 
 // Row m of a 32-row MFMA block reads key key_perm(m) of the block.  With the 32x32 C layout
 // (lane l, register i -> row (i/4)*8 + (l/32)*4 + i%4) this puts key (i/8)*16 + (l/32)*8 + i%8
@@ -736,7 +742,7 @@ void attn_kernel(AttnArgs args) {
       const float qn = a.q_rms[(int64_t)b * a.q_rms_sb + qrc];
 #pragma unroll
       for (int k = 0; k < 8; ++k) {
-        const Vec8<float> wk = Vec8<float>::load(qw + k * 16);
+        const Vec8<float> wk = load8_u(qw + k * 16);
 #pragma unroll
         for (int e = 0; e < 8; ++e) y[k].set(e, (float)qx[k].get(e) * qn * wk.get(e));
       }
@@ -1048,6 +1054,12 @@ void attn_kernel(AttnArgs args) {
       int tok0, key0, tj;
       if (tile_needs_mask(0, tok0, key0, tj)) mask_tile(s_cur, hh, tok0, tj, key0, lim_lane);
     }
+    // the running max starts at tile 0's own (what the rare path below would set on step 0, for
+    // every lane, after a wasted pass over the tile)
+    float mx = -INFINITY;
+#pragma unroll
+    for (int e = 0; e < 32; ++e) mx = fmaxf(mx, s_cur[e >> 4][e & 15]);
+    m_run = pair_max(mx) * c2;
     __syncthreads();  // K(0) read by every wave before its buffer takes K(kRing)
   }
 
@@ -1586,7 +1598,7 @@ void attn_fp8_kernel(AttnArgs args) {
       const float qn = a.q_rms[(int64_t)b * a.q_rms_sb + qrc];
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
-        const Vec8<float> wk = Vec8<float>::load(qw + (i >> 2) * 64 + (i & 3) * 8);
+        const Vec8<float> wk = load8_u(qw + (i >> 2) * 64 + (i & 3) * 8);
 #pragma unroll
         for (int j = 0; j < 8; ++j) qb[i].set(j, (bf16)((float)qx[i].get(j) * qn * wk.get(j)));
       }
@@ -1870,7 +1882,25 @@ void attn_fp8_kernel(AttnArgs args) {
     log_pv = __builtin_amdgcn_logf(pv);
     inv_pv = __builtin_amdgcn_rcpf(pv);
   };
-  if (ntau > 0) open_scales(w0.slot);
+  // the tile's max per query (both key halves), in log2 units
+  auto tile_max = [&](const f32x16 (&s)[2]) __attribute__((always_inline)) {
+    float mq[2];
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      const f32x16& sc = s[c];
+      mq[c] = max3_raw(sc[0], sc[1], sc[2]);
+#pragma unroll
+      for (int r = 3; r < 15; r += 2) mq[c] = max3_raw(mq[c], sc[r], sc[r + 1]);
+      mq[c] = max3_raw(mq[c], sc[15], sc[15]);
+    }
+    return pair_max_raw(max3_raw(mq[0], mq[1], mq[1])) * mult;
+  };
+  if (ntau > 0) {
+    open_scales(w0.slot);
+    // the running max starts at tile 0's own, which the rare path would set on step 1 after a
+    // wasted pass over the tile
+    m_run = fmaxf(m_run, tile_max(sA));
+  }
   int open_slot = -1;  // the slot of the frame the next tile opens (wave-uniform), else -1
   // Settles P of the previous tile (scores s) before its PV product.  Probabilities use the
   // running max m, not the tile's own max: an e4m3 probability at or above 480 converts to NaN,
@@ -1882,16 +1912,7 @@ void attn_fp8_kernel(AttnArgs args) {
     {
       // both key halves of a query take the same decision
       const bool needq = pair_max(need ? 1.f : 0.f) > 0.f;
-      float mq[2];
-#pragma unroll
-      for (int c = 0; c < 2; ++c) {
-        const f32x16& sc = s[c];
-        mq[c] = max3_raw(sc[0], sc[1], sc[2]);
-#pragma unroll
-        for (int r = 3; r < 15; r += 2) mq[c] = max3_raw(mq[c], sc[r], sc[r + 1]);
-        mq[c] = max3_raw(mq[c], sc[15], sc[15]);
-      }
-      const float mx = pair_max_raw(max3_raw(mq[0], mq[1], mq[1])) * mult;
+      const float mx = tile_max(s);
       const float m_new = needq ? fmaxf(m_run, mx) : m_run;
       const float alpha = m_new == m_run ? 1.0f : __builtin_amdgcn_exp2f(m_run - m_new);
       const float bias2 = log_pv - (m_new == -INFINITY ? 0.f : m_new);
