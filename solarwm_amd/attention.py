@@ -141,7 +141,9 @@ def norm_spec(norm, heads: int, device) -> tuple[torch.Tensor, float]:
         weight, eps = norm
     else:
         weight, eps = norm.weight, norm.eps
-    w = weight.detach().to(device=device, dtype=torch.float32).reshape(-1).contiguous()
+    w = weight
+    if w.dtype != torch.float32 or w.device != device or w.dim() != 1 or not w.is_contiguous():
+        w = w.detach().to(device=device, dtype=torch.float32).reshape(-1).contiguous()
     if w.numel() != heads * kernels.HEAD_DIM:
         raise ValueError(f"norm weight has {w.numel()} entries, expected {heads * kernels.HEAD_DIM}")
     return w, float(eps)

@@ -104,25 +104,32 @@ def dtype_code(dtype: torch.dtype) -> int:
         raise ValueError(f"unsupported dtype {dtype}; expected float32, bfloat16, float16 or float8_e4m3fn")
 
 
+def _device_index(device: torch.device) -> int:
+    return device.index if device.index is not None else torch.cuda.current_device()
+
+
 def _stream(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    # the raw handle: building a torch.cuda.Stream object for it costs 1.7 us a call
+    return torch._C._cuda_getCurrentRawStream(_device_index(device))
 
 
 def _require_cuda(name: str, t: torch.Tensor) -> None:
     if not isinstance(t, torch.Tensor):
         raise TypeError(f"{name} must be a torch.Tensor")
-    if t.device.type != "cuda":
+    if not t.is_cuda:
         raise ValueError(f"{name} must be a GPU tensor (got device {t.device})")
 
 
 def _token_major(name: str, t: torch.Tensor) -> tuple[int, int, int]:
     """Validate a [B, L, H, D] tensor with unit stride on D; return (sb, st, sh)."""
     _require_cuda(name, t)
-    if t.dim() != 4 or t.shape[-1] != HEAD_DIM:
-        raise ValueError(f"{name} must be [B, L, H, {HEAD_DIM}], got {tuple(t.shape)}")
-    if t.stride(-1) != 1:
+    shape = t.shape
+    if len(shape) != 4 or shape[3] != HEAD_DIM:
+        raise ValueError(f"{name} must be [B, L, H, {HEAD_DIM}], got {tuple(shape)}")
+    sb, st, sh, sd = t.stride()
+    if sd != 1:
         raise ValueError(f"{name} must be contiguous in its last dimension")
-    return t.stride(0), t.stride(1), t.stride(2)
+    return sb, st, sh
 
 
 def check_pools(kpool: torch.Tensor, vpool: torch.Tensor, frame_tokens: int) -> tuple[int, int, int]:
@@ -130,12 +137,13 @@ def check_pools(kpool: torch.Tensor, vpool: torch.Tensor, frame_tokens: int) -> 
     _require_cuda("k_pool", kpool)
     _require_cuda("v_pool", vpool)
     tp = padded_tokens(frame_tokens)
-    if kpool.dim() != 5 or vpool.dim() != 5:
+    kshape, vshape = kpool.shape, vpool.shape
+    if len(kshape) != 5 or len(vshape) != 5:
         raise ValueError("pools must be 5-D: K [S,B,H,Tp,D], V [S,B,H,D,Tp]")
-    s, b, h = kpool.shape[:3]
-    if tuple(kpool.shape) != (s, b, h, tp, HEAD_DIM) or tuple(vpool.shape) != (s, b, h, HEAD_DIM, tp):
+    s, b, h = kshape[:3]
+    if kshape != (s, b, h, tp, HEAD_DIM) or vshape != (s, b, h, HEAD_DIM, tp):
         raise ValueError(
-            f"pool shapes {tuple(kpool.shape)} / {tuple(vpool.shape)} do not match "
+            f"pool shapes {tuple(kshape)} / {tuple(vshape)} do not match "
             f"K [S,B,H,{tp},{HEAD_DIM}] / V [S,B,H,{HEAD_DIM},{tp}] for frame_tokens={frame_tokens}"
         )
     if not (kpool.is_contiguous() and vpool.is_contiguous()):
@@ -218,8 +226,7 @@ def workspace(device: torch.device, nbytes: int) -> tuple[int, int, torch.Tensor
     allocator has handed to another tensor."""
     if nbytes <= 0:
         return 0, 0, None
-    key = (device.index if device.index is not None else torch.cuda.current_device(),
-           _stream(device))
+    key = (_device_index(device), _stream(device))
     t = _workspaces.get(key)
     if t is None or t.numel() < nbytes:
         t = torch.empty(int(nbytes), dtype=torch.uint8, device=device)
@@ -497,7 +504,7 @@ def attention_desc(
         raise RuntimeError("attention over an empty key window")
     if out is None:
         out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
-    if tuple(out.shape) != tuple(q.shape) or out.dtype != q.dtype:
+    elif out.shape != q.shape or out.dtype != q.dtype:
         raise ValueError("out must match q's shape and dtype")
     osb, ost, osh = _token_major("out", out)
     scale = 1.0 / math.sqrt(HEAD_DIM) if softmax_scale is None else float(softmax_scale)
@@ -698,8 +705,7 @@ def staging_pools(
         raise ValueError("staging pools hold bf16, f16 or float32 frames")
     tp = padded_tokens(frame_tokens)
     n = n_slots * batch * heads * tp * HEAD_DIM
-    key = (device.index if device.index is not None else torch.cuda.current_device(),
-           _stream(device), dtype)
+    key = (_device_index(device), _stream(device), dtype)
     buf = _staging.get(key)
     if buf is None or buf.numel() < 2 * n:
         buf = torch.empty(2 * n, dtype=dtype, device=device)
