@@ -748,14 +748,23 @@ void attn_kernel(AttnArgs args) {
       for (int i = 0; i < 4; ++i) qps[i] = *reinterpret_cast<const f32x4_u*>(ps + 4 * i);
     }
   }
+  // RMSNorm factor of this row and its channel weights, with the same loads (in form_q for the
+  // split instances, whose segment loop has no registers for them: they would spill)
+  [[maybe_unused]] float qn = 0.f;
+  [[maybe_unused]] Vec8<float> qnw[8];
+  if (!SPLIT && a.q_rms) {
+    qn = a.q_rms[(int64_t)b * a.q_rms_sb + qrc];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) qnw[k] = load8_u(qw + k * 16);
+  }
   // qx -> qf (and qt0), once the tile loads are in flight
   auto form_q = [&]() __attribute__((always_inline)) {
     Vec8<float> y[8];
-    if (a.q_rms) {  // RMSNorm factor of this row and its channel weights
-      const float qn = a.q_rms[(int64_t)b * a.q_rms_sb + qrc];
+    if (a.q_rms) {
+      if (SPLIT) qn = a.q_rms[(int64_t)b * a.q_rms_sb + qrc];
 #pragma unroll
       for (int k = 0; k < 8; ++k) {
-        const Vec8<float> wk = load8_u(qw + k * 16);
+        const Vec8<float> wk = SPLIT ? load8_u(qw + k * 16) : qnw[k];
 #pragma unroll
         for (int e = 0; e < 8; ++e) y[k].set(e, (float)qx[k].get(e) * qn * wk.get(e));
       }
@@ -1604,15 +1613,24 @@ void attn_fp8_kernel(AttnArgs args) {
         }
     }
   }
+  // RMSNorm factor of this row and its channel weights, with the same loads (in form_q for the
+  // split instances, whose segment loop has no registers for them: they would spill)
+  [[maybe_unused]] float qn = 0.f;
+  [[maybe_unused]] Vec8<float> qnw[8];
+  if (!SPLIT && a.q_rms) {
+    qn = a.q_rms[(int64_t)b * a.q_rms_sb + qrc];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) qnw[i] = load8_u(qw + (i >> 2) * 64 + (i & 3) * 8);
+  }
   auto form_q = [&]() __attribute__((always_inline)) {
     // the row in bf16 throughout (bf16 inputs, or the norm's / RoPE's bf16 outputs): chunk i holds
     // channels (i >> 2) * 64 + 32 hh + 8 (i & 3) .. +7
     Vec8<bf16> qb[8];
     if (a.q_rms) {  // normalised Q in bf16, as the reference's norm_q output
-      const float qn = a.q_rms[(int64_t)b * a.q_rms_sb + qrc];
+      if (SPLIT) qn = a.q_rms[(int64_t)b * a.q_rms_sb + qrc];
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
-        const Vec8<float> wk = load8_u(qw + (i >> 2) * 64 + (i & 3) * 8);
+        const Vec8<float> wk = SPLIT ? load8_u(qw + (i >> 2) * 64 + (i & 3) * 8) : qnw[i];
 #pragma unroll
         for (int j = 0; j < 8; ++j) qb[i].set(j, (bf16)((float)qx[i].get(j) * qn * wk.get(j)));
       }
@@ -2645,6 +2663,21 @@ static int attention_impl(const void* q, int q_dtype, int64_t q_sb, int64_t q_st
         split_bytes = split_workspace_bytes(n_cu);
         split_mode = 2;
       }
+    }
+  }
+  // Unsplit grids that give every CU at most one workgroup either way: 4-wave groups spread the
+  // queries over twice the CUs and start sooner, which wins while the window is short (8 waves -> 4,
+  // us a launch: H24, 1215 queries x 512 keys 22.4 -> 17.4; H12, 1560 x 2048 50.7 -> 46.6; fp8 H24,
+  // 880 x 6160 99.5 -> 79.8; RoPE H12, 1760 x 98 tiles 136 -> 131); over long ones the 8-wave
+  // group's half as many staged bytes per query wins (H12, 1560 queries x 147 tiles 187 -> 191, x 512
+  // tiles 623 -> 648).  Up to 4 tiles they also win where they take two to a CU (H12, 4680 x 226 keys
+  // 18.7 -> 17.9; H16, 4000 x 77 16.4 -> 15.5; but 4680 x 512 keys 25.5 -> 26.9).
+  if (nw == 8 && n_segments == 0 && (split_bytes == 0 || workspace == nullptr)) {
+    const int64_t wg4 = (int64_t)((q_len + 127) / 128) * heads * batch;
+    if (nt <= 4 || (nt <= 100 && wg4 <= n_cu)) {
+      nw = 4;
+      a.n_qtiles = (q_len + 127) / 128;
+      a.n_wg = (int)wg4;
     }
   }
   // The split needs the caller's workspace (2 records of kSplitBQ rows x (O, max, sum) per

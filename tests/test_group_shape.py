@@ -1,0 +1,46 @@
+"""The workgroup shape of unsplit attention launches (``skv_attention_plan``, no GPU needed: 256 CUs):
+4-wave groups for short windows over grids that leave CUs idle, and for windows of up to 4 tiles; on
+the GPU, that the rows around 128-row groups come out as the oracle has them."""
+
+import pytest
+import torch
+
+from oracle import wan_cache_ref as ref
+from solarwm_amd import _lib, kernels
+
+from .helpers import assert_attn_close
+from .test_capi import _attn_desc, _plan
+
+
+@pytest.mark.parametrize("B,H,Lq,T,nf,pool,want", [
+    (1, 24, 1215, 512, 1, _lib.SKV_BF16, 4),    # 240 groups of 128 rows, 8 tiles
+    (1, 24, 1280, 640, 10, _lib.SKV_BF16, 4),   # 240 groups, 100 tiles
+    (1, 2, 16384, 6464, 1, _lib.SKV_BF16, 8),   # 256 groups, 101 tiles
+    (1, 2, 16385, 512, 1, _lib.SKV_BF16, 8),    # 258 groups
+    (1, 12, 4680, 512, 1, _lib.SKV_BF16, 8),    # 228 8-wave groups fill the chip
+    (1, 12, 4680, 256, 1, _lib.SKV_BF16, 4),    # 4 tiles
+    (1, 12, 4680, 257, 1, _lib.SKV_BF16, 8),    # 5 tiles
+    (1, 2, 128, 64, 5, _lib.SKV_FP8_E4M3, 4),
+])
+def test_waves_per_group(B, H, Lq, T, nf, pool, want):
+    d, _keep = _attn_desc(B, H, Lq, T, nf, pool)
+    plan = _plan(d)
+    rows = 32 * want
+    assert plan.waves_per_group == want and plan.split == 0
+    assert plan.n_workgroups == plan.n_qtiles == -(-Lq // rows) * H * B
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("H,Lq,T,nf", [(2, 1, 64, 1), (3, 127, 65, 2), (1, 129, 40, 3), (2, 257, 200, 4)])
+def test_small_grids(gpu, H, Lq, T, nf):
+    print("group shape", H, Lq, T, nf, flush=True)
+    g = torch.Generator().manual_seed(Lq)
+    q = torch.randn(1, Lq, H, 128, generator=g).bfloat16()
+    k, v = (torch.randn(1, nf * T, H, 128, generator=g).bfloat16() for _ in range(2))
+    kp, vp, _, _ = kernels.new_pools(nf, 1, H, T, torch.bfloat16, gpu)
+    kernels.append_frames(k.to(gpu), v.to(gpu), kp, vp, list(range(nf)), frame_tokens=T)
+    qd = q.to(gpu)
+    assert kernels.attention_plan(qd, kp, vp, list(range(nf)), frame_tokens=T)["waves_per_group"] == 4
+    out = kernels.attention_frames(qd, kp, vp, list(range(nf)), frame_tokens=T)
+    torch.cuda.synchronize()
+    assert_attn_close(out, ref.attention(q, k, v))
