@@ -355,6 +355,44 @@ typedef struct skv_launch_plan {
 int skv_attention_plan(const skv_attention_desc* desc, skv_launch_plan* plan);
 
 /*
+ * skv_prope_stage — the camera staging of one fused-PRoPE forward (causal_model.py:1948-2066), shared
+ * by all layers, in one launch.  The chunk's n_qframes frames have view matrices `view` (raw) and
+ * `view_t` (after the translation transform; the same pointer when linear) and intrinsics `ks`,
+ * float32, rows contiguous (4x4 / 3x3), with element strides per stream (_sb) and frame (_sf).
+ * Staged frame i (chunk frame first + i) goes to slot staged[i] of the camera store (store_view
+ * [n_slots][batch][16], store_k [..][9], store_inv [..][16] = P^-1), or takes over slot keep[i]'s
+ * camera when keep[i] >= 0.  Outputs, float32: kv_xform [n_staged][batch][16] = P^-1 of the staged
+ * frames; q_xform_t [batch][n_keys][n_qframes][11][16], q_xform_s and out_xform
+ * [batch][n_qframes][16] as skv_attention_prope takes them for the key frames `window` (slots) at
+ * temporal positions k_pos and query frames at q_pos0 + f * q_step; inv_freq: the 22 temporal
+ * frequencies.  Arithmetic in float64.
+ */
+typedef struct skv_prope_stage_desc {
+  const float* view;
+  int64_t view_sb, view_sf;
+  const float* view_t;
+  int64_t view_t_sb, view_t_sf;
+  const float* ks;
+  int64_t ks_sb, ks_sf;
+  float* store_view;
+  float* store_k;
+  float* store_inv;
+  int n_slots, batch, n_qframes, n_keys, n_staged, first;
+  int q_pos0, q_step;
+  const double* inv_freq;  /* host, 22 */
+  const int32_t* window;   /* host, n_keys */
+  const int32_t* k_pos;    /* host, n_keys */
+  const int32_t* staged;   /* host, n_staged */
+  const int32_t* keep;     /* host, n_staged */
+  float* kv_xform;
+  float* q_xform_t;
+  float* q_xform_s;
+  float* out_xform;
+} skv_prope_stage_desc;
+
+int skv_prope_stage(const skv_prope_stage_desc* desc, skv_stream_t stream);
+
+/*
  * H3 transforms (MiniMax-H3 backend).  H3's attention segments take rotate-half MM-RoPE on head
  * channels [0, 96) and its camera PRoPE on channels [96, 128) (eight 4-vectors per row, each
  * multiplied by the row's 4x4 matrix) before attention, and the output matrix on the attention

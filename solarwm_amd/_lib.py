@@ -84,6 +84,22 @@ class H3XformDesc(ctypes.Structure):
     ]
 
 
+class PropeStageDesc(ctypes.Structure):
+    """``skv_prope_stage_desc`` (include/solarkv.h), field for field."""
+
+    _fields_ = [
+        ("view", _vp), ("view_sb", _i64), ("view_sf", _i64),
+        ("view_t", _vp), ("view_t_sb", _i64), ("view_t_sf", _i64),
+        ("ks", _vp), ("ks_sb", _i64), ("ks_sf", _i64),
+        ("store_view", _vp), ("store_k", _vp), ("store_inv", _vp),
+        ("n_slots", _i32), ("batch", _i32), ("n_qframes", _i32), ("n_keys", _i32),
+        ("n_staged", _i32), ("first", _i32), ("q_pos0", _i32), ("q_step", _i32),
+        ("inv_freq", ctypes.POINTER(ctypes.c_double)), ("window", _i32p), ("k_pos", _i32p),
+        ("staged", _i32p), ("keep", _i32p),
+        ("kv_xform", _vp), ("q_xform_t", _vp), ("q_xform_s", _vp), ("out_xform", _vp),
+    ]
+
+
 class LaunchPlan(ctypes.Structure):
     """``skv_launch_plan`` (include/solarkv.h): the launch skv_attention_ex would make."""
 
@@ -143,6 +159,7 @@ SIGNATURES: dict[str, tuple] = {
     "skv_attention_ex_noalloc": (_i32, [ctypes.POINTER(AttentionDesc), _vp]),
     "skv_noalloc_init": (_i32, []),
     "skv_append_workspace_size": (_i32, [ctypes.POINTER(AppendDesc), ctypes.POINTER(_i64)]),
+    "skv_prope_stage": (_i32, [ctypes.POINTER(PropeStageDesc), _vp]),
     "skv_h3_rope_prope": (_i32, [ctypes.POINTER(H3XformDesc), _vp]),
 }
 

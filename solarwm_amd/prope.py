@@ -21,11 +21,14 @@ solar/backends/wan22/runtime/data.py:516-530), stored per frame slot next to the
 
 from __future__ import annotations
 
+import ctypes
+import functools
 from dataclasses import dataclass, field
 from typing import Any, Sequence
 
 import torch
 
+from . import _lib, kernels
 from .rope import TEMPORAL_PAIRS, _inv_freq
 
 GROUPS_T = TEMPORAL_PAIRS // 2  # 11 channel groups of 4 hold temporal RoPE pairs only
@@ -164,6 +167,87 @@ class CameraPass:
     camera: CameraCache = field(repr=False)
 
 
+def _kernel_stages(cam, vq, kq, staging, keep, off_f, window, qpos) -> bool:
+    """Whether ``skv_prope_stage`` takes this forward: GPU cameras of the store's shapes that need no
+    gradient, frame counts within its argument arrays, evenly spaced query positions (what the
+    position rules give), and no staged slot that another staged frame keeps its camera from."""
+    b, nb = cam.viewmats.shape[1], len(qpos)
+    return (cam.device.type == "cuda" and not (vq.requires_grad or kq.requires_grad)
+            and vq.shape == (b, nb, 4, 4) and kq.shape == (b, nb, 3, 3)
+            and 0 < len(window) <= _lib.SKV_MAX_FRAMES
+            and len(staging) <= min(_lib.SKV_MAX_APPEND_FRAMES, nb - off_f)
+            and len(set(staging)) == len(staging) and not set(staging) & set(keep)
+            and all(qpos[i] - qpos[i - 1] == qpos[1] - qpos[0] for i in range(1, nb)))
+
+
+@functools.lru_cache(maxsize=8)
+def _inv_freq_host(theta: float):
+    return (ctypes.c_double * TEMPORAL_PAIRS)(*_inv_freq(2 * TEMPORAL_PAIRS, theta).tolist())
+
+
+def _rows(t: torch.Tensor) -> torch.Tensor:
+    """``t`` [B, F, n, n] with contiguous matrices."""
+    return t if t.stride(-1) == 1 and t.stride(-2) == t.shape[-1] else t.contiguous()
+
+
+def _stage_kernel(cam, theta, vq, view_t, kq, staging, keep, off_f, window, qpos, kpos):
+    """The tables of :func:`_stage_tensors` and the camera store's update in one launch."""
+    b, nb, nk, n = vq.shape[0], len(qpos), len(window), len(staging)
+    same = view_t is vq
+    vq, kq = _rows(vq), _rows(kq)
+    view_t = vq if same else _rows(view_t)
+    sizes = [n * b * 16, b * nk * nb * GROUPS_T * 16, b * nb * 16, b * nb * 16]
+    flat = torch.empty(sum(sizes), dtype=torch.float32, device=cam.device)
+    kv, w, qs, qo = torch.split(flat, sizes)
+    kv, w = kv.view(n, b, 4, 4), w.view(b, nk, nb, GROUPS_T, 4, 4)
+    qs, qo = qs.view(b, nb, 4, 4), qo.view(b, nb, 4, 4)
+    freq, win, kp = _inv_freq_host(theta), _lib.int32_array(window), _lib.int32_array(kpos)
+    st, kp_old = _lib.int32_array(staging), _lib.int32_array(keep)
+    d = _lib.PropeStageDesc(
+        view=vq.data_ptr(), view_sb=vq.stride(0), view_sf=vq.stride(1), view_t=view_t.data_ptr(),
+        view_t_sb=view_t.stride(0), view_t_sf=view_t.stride(1), ks=kq.data_ptr(),
+        ks_sb=kq.stride(0), ks_sf=kq.stride(1), store_view=cam.viewmats.data_ptr(),
+        store_k=cam.ks.data_ptr(), store_inv=cam.p_inv.data_ptr(),
+        n_slots=cam.viewmats.shape[0], batch=b, n_qframes=nb, n_keys=nk, n_staged=n, first=off_f,
+        q_pos0=qpos[0], q_step=qpos[1] - qpos[0] if nb > 1 else 0, inv_freq=freq, window=win,
+        k_pos=kp, staged=st, keep=kp_old, kv_xform=kv.data_ptr() if n else None,
+        q_xform_t=w.data_ptr(), q_xform_s=qs.data_ptr(), out_xform=qo.data_ptr())
+    lib = _lib.load()
+    _lib.check("skv_prope_stage", lib.skv_prope_stage(ctypes.byref(d), kernels._stream(cam.device)))
+    return kv, w, qs, qo
+
+
+def _stage_tensors(cam, theta, vq, view_t, kq, staging, keep, off_f, window, qpos, kpos):
+    """Store the staged frames' cameras and return (P⁻¹ of the staged frames, W per key frame, query
+    frame and temporal group, P_qᵀ, P_q) as tensor operations (any device)."""
+    dev = cam.device
+    b = vq.shape[0]
+    p_q, p_q_inv = projection(view_t, kq)  # [B, nb, 4, 4]
+    if staging:
+        new_view = vq.transpose(0, 1)[off_f : off_f + len(staging)].clone()  # [n, B, 4, 4]
+        new_k = kq.transpose(0, 1)[off_f : off_f + len(staging)].clone()
+        new_inv = p_q_inv.transpose(0, 1)[off_f : off_f + len(staging)].to(torch.float32)
+        for i, old in enumerate(keep):
+            if old >= 0:  # keep the previous camera of this position
+                new_view[i], new_k[i], new_inv[i] = cam.viewmats[old], cam.ks[old], cam.p_inv[old]
+        idx = torch.tensor(list(staging), dtype=torch.long, device=dev)
+        cam.viewmats.index_copy_(0, idx, new_view)
+        cam.ks.index_copy_(0, idx, new_k)
+        cam.p_inv.index_copy_(0, idx, new_inv.contiguous())
+        kv_xform = new_inv.contiguous()
+    else:
+        kv_xform = torch.zeros(0, b, 4, 4, dtype=torch.float32, device=dev)
+    widx = torch.tensor(list(window), dtype=torch.long, device=dev)
+    pk_inv = cam.p_inv.index_select(0, widx).to(torch.float64)  # [nk, B, 4, 4]
+    a = torch.einsum("bfik,jbkl->bfjil", p_q, pk_inv)  # P_q P_k⁻¹: [B, nb, nk, 4, 4]
+    rq = _temporal_rotations(qpos, theta, dev)  # [nb, 11, 4, 4]
+    rk = _temporal_rotations(kpos, theta, dev)  # [nk, 11, 4, 4]
+    # W = R_kᵀ Aᵀ R_q:  W_im = sum_{k,l} Rk_ki A_lk Rq_lm
+    w = torch.einsum("jgki,bfjlk,fglm->bjfgim", rk, a, rq)
+    return (kv_xform, w.to(torch.float32).contiguous(),
+            p_q.transpose(-1, -2).to(torch.float32).contiguous(), p_q.to(torch.float32).contiguous())
+
+
 def stage_camera_cache(kv_cache: Sequence[Any], cam_viewmats: torch.Tensor, cam_K: torch.Tensor,
                        current_start: int, num_new_tokens: int, *,
                        sink_recache_after_switch: bool = False, per_frame: bool = False,
@@ -203,8 +287,7 @@ def stage_camera_cache(kv_cache: Sequence[Any], cam_viewmats: torch.Tensor, cam_
     kq = kq.to(device=dev, dtype=torch.float32)
     cam.active = True  # camera-conditioned frames from here on (causal_model.py:2005-2019)
     c0.metadata_present = True  # a dropped camera state is recreated (causal_model.py:2008-2011)
-    tr = cam.cfg.camera_translation_transform
-    p_q, p_q_inv = projection(transform_relative_viewmats(vq, tr), kq)  # [B, nb, 4, 4]
+    view_t = transform_relative_viewmats(vq, cam.cfg.camera_translation_transform)
 
     # written frames: position ws_f + i takes chunk frame roped_offset/T + i, except positions
     # below the camera write start, which keep the camera already there
@@ -216,41 +299,20 @@ def stage_camera_cache(kv_cache: Sequence[Any], cam_viewmats: torch.Tensor, cam_
     if plan.action == "roll_and_insert" and plan.num_rolled_tokens > 0:
         sf, ef, rf = plan.sink_tokens // T, plan.num_evicted_tokens // T, plan.num_rolled_tokens // T
         pre[sf : sf + rf] = pre[sf + ef : sf + ef + rf]
-    if staging:
-        new_view = vq.transpose(0, 1)[off_f : off_f + len(staging)].clone()  # [n, B, 4, 4]
-        new_k = kq.transpose(0, 1)[off_f : off_f + len(staging)].clone()
-        new_inv = p_q_inv.transpose(0, 1)[off_f : off_f + len(staging)].to(torch.float32)
-        for i, s in enumerate(staging):
-            pos = ws_f + i
-            if pos * T < cam_ws:  # keep the previous camera of this position
-                old = pre[pos]
-                new_view[i], new_k[i], new_inv[i] = cam.viewmats[old], cam.ks[old], cam.p_inv[old]
-        idx = torch.tensor(list(staging), dtype=torch.long, device=dev)
-        cam.viewmats.index_copy_(0, idx, new_view)
-        cam.ks.index_copy_(0, idx, new_k)
-        cam.p_inv.index_copy_(0, idx, new_inv.contiguous())
-        kv_xform = new_inv.contiguous()
-    else:
-        kv_xform = torch.zeros(0, g.batch, 4, 4, dtype=torch.float32, device=dev)
+    keep = [pre[ws_f + i] if (ws_f + i) * T < cam_ws else -1 for i in range(len(staging))]
 
     from .attention import window_positions  # the RoPE positions attend_cached uses
 
     nb = num_new_tokens // T
     qpos, kpos = window_positions(c0, plan, window, nb, int(current_start))
-    widx = torch.tensor(list(window), dtype=torch.long, device=dev)
-    pk_inv = cam.p_inv.index_select(0, widx).to(torch.float64)  # [nk, B, 4, 4]
-    a = torch.einsum("bfik,jbkl->bfjil", p_q, pk_inv)  # P_q P_k⁻¹: [B, nb, nk, 4, 4]
-    theta = c0.rope.cfg.theta
-    rq = _temporal_rotations(qpos, theta, dev)  # [nb, 11, 4, 4]
-    rk = _temporal_rotations(kpos, theta, dev)  # [nk, 11, 4, 4]
-    # W = R_kᵀ Aᵀ R_q:  W_im = sum_{k,l} Rk_ki A_lk Rq_lm
-    w = torch.einsum("jgki,bfjlk,fglm->bjfgim", rk, a, rq)
+    stage = (_stage_kernel if _kernel_stages(cam, vq, kq, staging, keep, off_f, window, qpos)
+             else _stage_tensors)
+    kv_xform, w, qs, qo = stage(cam, c0.rope.cfg.theta, vq, view_t, kq, staging, keep, off_f, window,
+                                qpos, kpos)
     return CameraPass(
         current_start=int(current_start), num_new_tokens=int(num_new_tokens),
-        staging=tuple(staging), window=tuple(window), kv_xform=kv_xform,
-        q_xform_t=w.to(torch.float32).contiguous(),
-        q_xform_s=p_q.transpose(-1, -2).to(torch.float32).contiguous(),
-        out_xform=p_q.to(torch.float32).contiguous(), camera=cam)
+        staging=tuple(staging), window=tuple(window), kv_xform=kv_xform, q_xform_t=w,
+        q_xform_s=qs, out_xform=qo, camera=cam)
 
 
 def commit_camera_cache(update: CameraPass | None) -> None:
