@@ -95,7 +95,7 @@ struct AttnArgs {
   // stored in partly filled slots); keys t >= flen[j] of frame j are masked.  32-bit so a
   // wave-uniform index reads it with a scalar load.
   int32_t flen[SKV_MAX_FRAMES];
-  // Balanced key split (no mask, 8-wave groups): the n_wg workgroups share the
+  // Balanced key split (no mask, 8-wave groups): n_wg workgroups (of a grid of one per CU) share the
   // units = B*H*n_qtiles*nt (q-tile, key tile) pairs equally; workgroup i takes units
   // [i*units/n_wg, (i+1)*units/n_wg) in q-tile order (share_begin).  A q-tile that one workgroup
   // covers whole is written directly; a part of a split q-tile goes to record 2i (the
@@ -643,6 +643,7 @@ void attn_kernel(AttnArgs args) {
   {
     const int bid = blockIdx.x, xcd = bid & 7, idx = bid >> 3;
     const int per = args.n_wg >> 3, rem = args.n_wg & 7;
+    if (SPLIT && idx >= per + (xcd < rem)) return;  // a grid of one workgroup per CU, fewer shares
     logical = xcd * per + min(xcd, rem) + idx;
   }
   // Segments: key tiles [tb, te) of q-tile qg; one whole q-tile unless split.  A split share
@@ -1545,6 +1546,7 @@ void attn_fp8_kernel(AttnArgs args) {
   {
     const int bid = blockIdx.x, xcd = bid & 7, idx = bid >> 3;
     const int per = args.n_wg >> 3, rem = args.n_wg & 7;
+    if (SPLIT && idx >= per + (xcd < rem)) return;  // a grid of one workgroup per CU, fewer shares
     logical = xcd * per + min(xcd, rem) + idx;
   }
   // Segments: key tiles [tb, te) of q-tile qg, as in attn_kernel (one whole q-tile unless split;
@@ -2250,7 +2252,7 @@ static int64_t split_workspace_bytes(int n_wg) {
 
 template <int NW>
 static void launch(const AttnArgs& a, int q_dtype, int pool_dtype, int rm, hipStream_t s) {
-  dim3 grid(a.n_wg), block(NW * 64);
+  dim3 grid(a.split ? cu_count() : a.n_wg), block(NW * 64);
   if (pool_dtype == SKV_F16) {  // plain attention, f16 MFMAs; q f16 or f32 (checked by the caller)
     const bool qh = q_dtype == SKV_F16;
     if constexpr (NW == 8) {
@@ -2623,7 +2625,8 @@ static int attention_impl(const void* q, int q_dtype, int64_t q_sb, int64_t q_st
   }
   a.n_wg = a.n_qtiles * heads * batch;
   // Balanced key split: when the grid leaves many CUs idle (few q-tiles, e.g. one frame of
-  // queries), one 8-wave workgroup per CU takes an equal share of all (q-tile, key tile) units;
+  // queries), one 8-wave workgroup per CU (or nearly, split_shares below) takes an equal share of
+  // all (q-tile, key tile) units;
   // split q-tiles are merged by attn_combine_kernel.  A tile costs more the more CUs are busy
   // (measured on MI355X with 525 tiles per workgroup: 128, 224 and 256 busy CUs take 0.81, 0.92
   // and 1.0 of the full-chip time), modelled as t(busy) ~ 1 + 0.62 * busy / n_cu; the split
@@ -2665,6 +2668,21 @@ static int attention_impl(const void* q, int q_dtype, int64_t q_sb, int64_t q_st
       }
     }
   }
+  // Shares of a split over n_q q-tiles: one per CU, or, when they are not much longer for it, as
+  // many as divide every q-tile evenly, so that no share crosses from one q-tile into the next.
+  // A share that does pays a second start (query, first tiles) and a second record: some 8 us a
+  // launch for the bf16 instances, 18 for fp8.  What the longer shares cost against that is their
+  // extra tiles, nt / m - n_q nt / n_cu.  One share a CU -> even shares, us a launch: bf16 H12,
+  // 1560 queries x 147 tiles (84 q-tiles, 252 shares, 0.8 extra tiles) 117.4 -> 107.8; H24, 1215 x 126
+  // (240 shares, 3.9) 136.4 -> 129.4; 44 q-tiles x 289 (220, 8.1) 141.4 -> 139.8; but 72 x 289 (216,
+  // 15) 210.7 -> 211.4 and 105 x 289 (210, 26) 291.9 -> 303.1.  fp8: H12, 1560 x 525 223 -> 205; 66 x
+  // 294 (198, 22) 145.7 -> 137.0; 105 x 294 (210, 26) 201.5 -> 197.3; but 95 x 525 (190, 68) 251.7
+  // -> 261.5, and RoPE, 96 x 294 (192, 37) 184 -> 191 a layer pass.
+  const bool mfma8 = pool_dtype == SKV_FP8_E4M3 && !prope && !(rope && frame_tokens < kTile);
+  auto split_shares = [&](int64_t n_q) -> int {
+    const int64_t m = n_cu / n_q, wg = m * n_q;
+    return m >= 2 && (int64_t)nt * (n_cu - wg) <= (mfma8 ? 24 : 9) * m * n_cu ? (int)wg : n_cu;
+  };
   // Unsplit grids that give every CU at most one workgroup either way: 4-wave groups spread the
   // queries over twice the CUs and start sooner, which wins while the window is short (8 waves -> 4,
   // us a launch: H24, 1215 queries x 512 keys 22.4 -> 17.4; H12, 1560 x 2048 50.7 -> 46.6; fp8 H24,
@@ -2696,9 +2714,9 @@ static int attention_impl(const void* q, int q_dtype, int64_t q_sb, int64_t q_st
       nw = 8;
       a.split = 1;
       a.n_qtiles = (int)(qt8 / ((int64_t)heads * batch));
-      a.n_wg = n_cu;
-      a.share_base = (int)(units8 / n_cu);
-      a.share_rem = (int)(units8 % n_cu);
+      a.n_wg = split_shares(qt8);
+      a.share_base = (int)(units8 / a.n_wg);
+      a.share_rem = (int)(units8 % a.n_wg);
     } else {
       a.split = 2;  // launched below as an unsplit grid of the full rounds, then the tail
     }
@@ -2735,7 +2753,7 @@ static int attention_impl(const void* q, int q_dtype, int64_t q_sb, int64_t q_st
   }
   const int64_t full_wg = a.split == 2 ? (int64_t)(a.n_wg / n_cu) * n_cu : 0;
   if (plan) {
-    *plan = skv_launch_plan{nw, a.split, a.split == 2 ? (int)full_wg + n_cu : a.n_wg,
+    *plan = skv_launch_plan{nw, a.split, a.split == 2 ? (int)full_wg + n_cu : a.split ? n_cu : a.n_wg,
                             a.n_qtiles * heads * batch, split_bytes, a.nt};
     return SKV_OK;
   }
@@ -2764,9 +2782,9 @@ static int attention_impl(const void* q, int q_dtype, int64_t q_sb, int64_t q_st
     launch<8>(m, q_dtype, pool_dtype, rm, s);
     AttnArgs t = a;
     t.split = 1;
-    t.n_wg = n_cu;
-    t.share_base = n_tail * nt / n_cu;
-    t.share_rem = n_tail * nt % n_cu;
+    t.n_wg = split_shares(n_tail);
+    t.share_base = n_tail * nt / t.n_wg;
+    t.share_rem = n_tail * nt % t.n_wg;
     t.qt_base = (int)full_wg;
     launch<8>(t, q_dtype, pool_dtype, rm, s);
     combine(t, n_tail);
