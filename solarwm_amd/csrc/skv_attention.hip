@@ -2677,7 +2677,9 @@ static int attention_impl(const void* q, int q_dtype, int64_t q_sb, int64_t q_st
   // (240 shares, 3.9) 136.4 -> 129.4; 44 q-tiles x 289 (220, 8.1) 141.4 -> 139.8; but 72 x 289 (216,
   // 15) 210.7 -> 211.4 and 105 x 289 (210, 26) 291.9 -> 303.1.  fp8: H12, 1560 x 525 223 -> 205; 66 x
   // 294 (198, 22) 145.7 -> 137.0; 105 x 294 (210, 26) 201.5 -> 197.3; but 95 x 525 (190, 68) 251.7
-  // -> 261.5, and RoPE, 96 x 294 (192, 37) 184 -> 191 a layer pass.
+  // -> 261.5, and RoPE, 96 x 294 (192, 37) 184 -> 191 a layer pass
+  // (108 x 294, 216 shares, 23: 199 -> 196).  Tail launch of 60 q-tiles x 63 after three rounds: bf16
+  // 452 -> 446, fp8 382 -> 368.
   const bool mfma8 = pool_dtype == SKV_FP8_E4M3 && !prope && !(rope && frame_tokens < kTile);
   auto split_shares = [&](int64_t n_q) -> int {
     const int64_t m = n_cu / n_q, wg = m * n_q;
