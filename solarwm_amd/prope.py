@@ -27,6 +27,7 @@ from dataclasses import dataclass, field
 from typing import Any, Sequence
 
 import torch
+from torch.autograd import forward_ad
 
 from . import _lib, kernels
 from .rope import TEMPORAL_PAIRS, _inv_freq
@@ -167,12 +168,23 @@ class CameraPass:
     camera: CameraCache = field(repr=False)
 
 
+def _plain(t: torch.Tensor) -> bool:
+    """Whether a raw pointer tells all of ``t``: nothing that follows the operations on it (autograd
+    in either direction, function transforms, fake or traced tensors) would lose them."""
+    return (type(t) in (torch.Tensor, torch.nn.Parameter) and not t.requires_grad and not t.is_neg()
+            and not torch._C._functorch.is_functorch_wrapped_tensor(t)
+            and forward_ad.unpack_dual(t).tangent is None)
+
+
 def _kernel_stages(cam, vq, kq, staging, keep, off_f, window, qpos) -> bool:
-    """Whether ``skv_prope_stage`` takes this forward: GPU cameras of the store's shapes that need no
-    gradient, frame counts within its argument arrays, evenly spaced query positions (what the
-    position rules give), and no staged slot that another staged frame keeps its camera from."""
+    """Whether ``skv_prope_stage`` takes this forward: GPU cameras of the store's shapes that nothing
+    follows (nor the store's own), frame counts within its argument arrays, evenly spaced query
+    positions (what the position rules give), and no staged slot that another staged frame keeps its
+    camera from."""
     b, nb = cam.viewmats.shape[1], len(qpos)
-    return (cam.device.type == "cuda" and not (vq.requires_grad or kq.requires_grad)
+    return (cam.device.type == "cuda"
+            and all(_plain(t) for t in (vq, kq, cam.viewmats, cam.ks, cam.p_inv))
+            and not torch.jit.is_tracing() and torch._C._len_torch_dispatch_stack() == 0
             and vq.shape == (b, nb, 4, 4) and kq.shape == (b, nb, 3, 3)
             and 0 < len(window) <= _lib.SKV_MAX_FRAMES
             and len(staging) <= min(_lib.SKV_MAX_APPEND_FRAMES, nb - off_f)

@@ -7,6 +7,8 @@ import ctypes
 
 import pytest
 import torch
+from torch._subclasses import FakeTensorMode
+from torch.fx.experimental.proxy_tensor import make_fx
 
 from solarwm_amd import PropeConfig, RopeConfig, _lib, make_kv_cache_allocator, prope, stage_camera_cache
 
@@ -83,6 +85,32 @@ def test_stage_kernel_takes_strided_cameras(gpu):
             assert torch.equal(getattr(got, name), getattr(want, name))
 
 
+@pytest.mark.gpu
+def test_followed_cameras_keep_what_follows_them(gpu):
+    """Forward-mode tangents reach the four tables, and the gradients of cameras staged earlier reach
+    the tables of later forwards through the store."""
+    fwd = torch.autograd.forward_ad
+    vm, ks = (x.to(gpu) for x in trajectory(1, 4, seed=3))
+    tables = ("kv_xform", "q_xform_t", "q_xform_s", "out_xform")
+    want = stage_camera_cache(_caches(gpu, 1, 5, 0, 2, "logd4", True), vm, ks, 0, 2 * T, per_frame=True)
+    with fwd.dual_level():
+        dual = fwd.make_dual(vm, torch.randn_like(vm))
+        got = stage_camera_cache(_caches(gpu, 1, 5, 0, 2, "logd4", True), dual, ks, 0, 2 * T, per_frame=True)
+        for name in tables:
+            x = fwd.unpack_dual(getattr(got, name))
+            assert x.tangent is not None and float(x.tangent.abs().max()) > 0, name
+            _close(x.primal, getattr(want, name))
+    caches = _caches(gpu, 1, 5, 0, 2, "linear", True)
+    first = vm[:, :2].clone().requires_grad_()
+    stage_camera_cache(caches, first, ks[:, :2], 0, 2 * T, per_frame=True)
+    c = caches[0]
+    plan, temp, _, _ = c.plan(0, 2 * T, False)
+    c.commit(c.stage(plan, temp), plan.current_end, plan.local_end_index)
+    later = stage_camera_cache(caches, vm, ks, 2 * T, 2 * T, per_frame=True)
+    (grad,) = torch.autograd.grad(later.q_xform_t.sum(), first)
+    assert float(grad.abs().max()) > 0
+
+
 def test_stage_rule_and_refusals():
     cam = prope.CameraCache(8, 2, "cpu", PropeConfig())
     v, k = torch.zeros(2, 3, 4, 4), torch.zeros(2, 3, 3, 3)
@@ -97,6 +125,27 @@ def test_stage_rule_and_refusals():
     assert not rule(keep=(-1, -1, 4)) and not rule(staging=(4, 5, 5)) and not rule(qpos=(5, 6, 8))
     assert not rule(window=()) and not rule(window=range(257))
     assert not rule(v=v.clone().requires_grad_())
+
+
+    # cameras, or a store, that something follows: the launch would lose it
+    with torch.autograd.forward_ad.dual_level():
+        dual = torch.autograd.forward_ad.make_dual(v, torch.ones_like(v))
+        assert not rule(v=dual) and not rule(k=torch.autograd.forward_ad.make_dual(k, torch.ones_like(k)))
+    seen = []
+    torch.func.vmap(lambda x: (seen.append(rule(v=x)), x)[1])(v[None])
+    torch.func.jvp(lambda x: (seen.append(rule(k=x)), x)[1], (k,), (k,))
+    make_fx(lambda x: (seen.append(rule(v=x)), x + 1)[1])(v)
+    with FakeTensorMode() as fake:
+        seen.append(rule())
+        seen.append(rule(v=fake.from_tensor(v)))
+    assert seen == [False] * 5 and rule()
+    assert not rule(v=torch._neg_view(v))
+    for name in ("viewmats", "ks", "p_inv"):
+        t = getattr(cam, name)
+        setattr(cam, name, t.clone().requires_grad_())
+        assert not rule(), name
+        setattr(cam, name, t)
+    assert rule()
 
     lib = _lib.load()
     buf = (ctypes.c_float * 64)()
