@@ -178,11 +178,11 @@ def _plain(t: torch.Tensor) -> bool:
 
 def _kernel_stages(cam, vq, kq, staging, keep, off_f, window, qpos) -> bool:
     """Whether ``skv_prope_stage`` takes this forward: GPU cameras of the store's shapes that nothing
-    follows (nor the store's own), frame counts within its argument arrays, evenly spaced query
-    positions (what the position rules give), and no staged slot that another staged frame keeps its
-    camera from."""
+    follows (nor the store's own), a chunk of at least one frame, frame counts within its argument
+    arrays, evenly spaced query positions (what the position rules give), and no staged slot that
+    another staged frame keeps its camera from."""
     b, nb = cam.viewmats.shape[1], len(qpos)
-    return (cam.device.type == "cuda"
+    return (cam.device.type == "cuda" and 0 < b <= 65535 and 0 < nb  # grid (key frames + 1, b)
             and all(_plain(t) for t in (vq, kq, cam.viewmats, cam.ks, cam.p_inv))
             and not torch.jit.is_tracing() and torch._C._len_torch_dispatch_stack() == 0
             and vq.shape == (b, nb, 4, 4) and kq.shape == (b, nb, 3, 3)

@@ -86,6 +86,22 @@ def test_stage_kernel_takes_strided_cameras(gpu):
 
 
 @pytest.mark.gpu
+def test_staging_without_new_frames(gpu):
+    """A call without new frames over a committed history gives empty query tables, as on the CPU."""
+    vm, ks = trajectory(2, 2, seed=5)
+    shapes = []
+    for dev in (gpu, torch.device("cpu")):
+        caches = _caches(dev, 2, 6, 1, 2, "linear", True)
+        stage_camera_cache(caches, vm.to(dev), ks.to(dev), 0, 2 * T, per_frame=True)
+        c = caches[0]
+        plan, temp, _, _ = c.plan(0, 2 * T, False)
+        c.commit(c.stage(plan, temp), plan.current_end, plan.local_end_index)
+        got = stage_camera_cache(caches, vm.to(dev), ks.to(dev), 2 * T, 0, per_frame=True)
+        shapes.append([tuple(getattr(got, n).shape) for n in ("kv_xform", "q_xform_t", "q_xform_s", "out_xform")])
+    assert shapes[0] == shapes[1] and shapes[0][1] == (2, 2, 0, 11, 4, 4)
+
+
+@pytest.mark.gpu
 def test_followed_cameras_keep_what_follows_them(gpu):
     """Forward-mode tangents reach the four tables, and the gradients of cameras staged earlier reach
     the tables of later forwards through the store."""
@@ -123,6 +139,11 @@ def test_stage_rule_and_refusals():
     assert rule() and rule(qpos=(5, 5, 5))
     assert not rule(v=v[:1]) and not rule(k=torch.zeros(2, 3, 4, 4)) and not rule(off=1)
     assert not rule(keep=(-1, -1, 4)) and not rule(staging=(4, 5, 5)) and not rule(qpos=(5, 6, 8))
+    assert not rule(v=v[:, :0], k=k[:, :0], staging=(), keep=(), qpos=())  # no new frames
+    wide = prope.CameraCache(1, 65536, "cpu", PropeConfig())
+    wide.device = cam.device
+    assert not prope._kernel_stages(wide, v[:1, :1].expand(65536, 1, 4, 4), k[:1, :1].expand(65536, 1, 3, 3),
+                                    [0], [-1], 0, [0], [0])
     assert not rule(window=()) and not rule(window=range(257))
     assert not rule(v=v.clone().requires_grad_())
 
