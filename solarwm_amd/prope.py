@@ -186,6 +186,7 @@ def _kernel_stages(cam, vq, kq, staging, keep, off_f, window, qpos) -> bool:
             and all(_plain(t) for t in (vq, kq, cam.viewmats, cam.ks, cam.p_inv))
             and not torch.jit.is_tracing() and torch._C._len_torch_dispatch_stack() == 0
             and vq.shape == (b, nb, 4, 4) and kq.shape == (b, nb, 3, 3)
+            and vq.device == kq.device == cam.p_inv.device
             and 0 < len(window) <= _lib.SKV_MAX_FRAMES
             and len(staging) <= min(_lib.SKV_MAX_APPEND_FRAMES, nb - off_f)
             and len(set(staging)) == len(staging) and not set(staging) & set(keep)
@@ -209,7 +210,8 @@ def _stage_kernel(cam, theta, vq, view_t, kq, staging, keep, off_f, window, qpos
     vq, kq = _rows(vq), _rows(kq)
     view_t = vq if same else _rows(view_t)
     sizes = [n * b * 16, b * nk * nb * GROUPS_T * 16, b * nb * 16, b * nb * 16]
-    flat = torch.empty(sum(sizes), dtype=torch.float32, device=cam.device)
+    dev = cam.p_inv.device
+    flat = torch.empty(sum(sizes), dtype=torch.float32, device=dev)
     kv, w, qs, qo = torch.split(flat, sizes)
     kv, w = kv.view(n, b, 4, 4), w.view(b, nk, nb, GROUPS_T, 4, 4)
     qs, qo = qs.view(b, nb, 4, 4), qo.view(b, nb, 4, 4)
@@ -225,7 +227,8 @@ def _stage_kernel(cam, theta, vq, view_t, kq, staging, keep, off_f, window, qpos
         k_pos=kp, staged=st, keep=kp_old, kv_xform=kv.data_ptr() if n else None,
         q_xform_t=w.data_ptr(), q_xform_s=qs.data_ptr(), out_xform=qo.data_ptr())
     lib = _lib.load()
-    _lib.check("skv_prope_stage", lib.skv_prope_stage(ctypes.byref(d), kernels._stream(cam.device)))
+    with torch.cuda.device(dev):  # a launch goes to the current device, tensor operations to their tensors'
+        _lib.check("skv_prope_stage", lib.skv_prope_stage(ctypes.byref(d), kernels._stream(dev)))
     return kv, w, qs, qo
 
 

@@ -131,7 +131,7 @@ def test_stage_rule_and_refusals():
     cam = prope.CameraCache(8, 2, "cpu", PropeConfig())
     v, k = torch.zeros(2, 3, 4, 4), torch.zeros(2, 3, 3, 3)
     assert not prope._kernel_stages(cam, v, k, [0], [-1], 0, [0], [0, 1, 2])  # CPU cameras
-    cam.device = torch.device("cuda", 0)  # the rule reads sizes only
+    cam.device = torch.device("cuda", 0)  # the rule reads sizes and marks only
 
     def rule(v=v, k=k, staging=(4, 5, 6), keep=(-1, -1, 2), off=0, window=(0, 4), qpos=(5, 6, 7)):
         return prope._kernel_stages(cam, v, k, staging, keep, off, window, qpos)
@@ -139,6 +139,7 @@ def test_stage_rule_and_refusals():
     assert rule() and rule(qpos=(5, 5, 5))
     assert not rule(v=v[:1]) and not rule(k=torch.zeros(2, 3, 4, 4)) and not rule(off=1)
     assert not rule(keep=(-1, -1, 4)) and not rule(staging=(4, 5, 5)) and not rule(qpos=(5, 6, 8))
+    assert not rule(v=v.to("meta")) and not rule(k=k.to("meta"))  # on another device than the store
     assert not rule(v=v[:, :0], k=k[:, :0], staging=(), keep=(), qpos=())  # no new frames
     wide = prope.CameraCache(1, 65536, "cpu", PropeConfig())
     wide.device = cam.device
@@ -188,6 +189,35 @@ def test_stage_rule_and_refusals():
                  dict(keep=[4]), dict(keep=[1]), dict(n_staged=2, staged=[1, 1], keep=[-1, -1])):
         assert call(**over) == _lib.SKV_E_ARG, over
     assert lib.skv_prope_stage(None, None) == _lib.SKV_E_ARG
+
+
+def test_stage_launch_runs_on_the_cameras_device(monkeypatch):
+    """The launch is made with the store's device current, whatever device the caller has current."""
+    current, launched = [], []
+
+    class Device:
+        def __init__(self, dev):
+            self.dev = dev
+
+        def __enter__(self):
+            current.append(self.dev)
+
+        def __exit__(self, *a):
+            current.pop()
+
+    class Lib:
+        @staticmethod
+        def skv_prope_stage(desc, stream):
+            launched.append((list(current), stream))
+            return _lib.SKV_OK
+
+    monkeypatch.setattr(torch.cuda, "device", Device)
+    monkeypatch.setattr(prope.kernels, "_stream", lambda dev: ("stream of", dev))
+    monkeypatch.setattr(prope._lib, "load", lambda: Lib)
+    cam = prope.CameraCache(8, 2, "cpu", PropeConfig())
+    v, k = torch.zeros(2, 3, 4, 4), torch.zeros(2, 3, 3, 3)
+    prope._stage_kernel(cam, 1e4, v, v, k, [4], [-1], 0, [0, 4], [1, 2, 3], [0, 1])
+    assert launched == [([cam.p_inv.device], ("stream of", cam.p_inv.device))]
 
 
 def test_stage_descriptor_layout(tmp_path):
