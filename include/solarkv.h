@@ -12,8 +12,9 @@
  *     2 x n_cu x 256 rows x 130 floats, 68 MB on 256 CUs);
  *   - an fp8 append of a chunk with fewer than 4 (frame, batch, head, K|V) units per CU takes
  *     the one-pass slice kernel (bf16 sources, no K norm, 8-byte aligned workspace: a 128 B
- *     header + 512 B per unit) or else the tile-grid kernels (one float per 64-token tile);
- *     skv_append_workspace_size reports the larger of the two.
+ *     header + 512 B per unit) or else the tile-grid kernels (one float per 64-token tile); with
+ *     RoPE / PRoPE copies it takes the tile grids (two floats per tile), raw frames and copies
+ *     together.  skv_append_workspace_size reports the largest of these that applies.
  * Without a workspace the same calls run the unsplit kernels (same results up to fp32
  * summation order for attention; bit-identical for the append).  A workspace is read and
  * written by the launch on `stream` only, so one workspace serves any number of calls on one
@@ -249,7 +250,8 @@ typedef struct skv_append_desc {
   void* vx_pool;
   const float* kv_xform;
   void* workspace;         /* device, optional, 4-byte aligned (8 for the one-pass fp8 kernel) */
-  int64_t workspace_bytes; /* its size; must cover skv_append_workspace_size */
+  int64_t workspace_bytes; /* its size, skv_append_workspace_size (from one float per tile on, copies
+                              with a smaller one run after the raw frames) */
   float* kr_scale;         /* fp8 pools with kr_pool */
   float* vx_scale;         /* fp8 pools with vx_pool */
 } skv_append_desc;

@@ -8,6 +8,7 @@
 // (frame, batch, head); K rows move as 16 B vectors, V is transposed in registers, 8 tokens x 8
 // channels per thread, so the pool keeps V channel-major (tokens contiguous), which is what the
 // attention kernel's PV product reads.
+#include <algorithm>
 #include <cstdlib>
 
 #include "skv_common.h"
@@ -1339,12 +1340,15 @@ static int append_impl(const void* k_new, const void* v_new, int src_dtype, int6
   const int64_t tile_bytes = few_units ? (int64_t)units * a.ntiles * (int64_t)sizeof(float) : 0;
   const int64_t cell_bytes = few_units ? (kSliceHead + (int64_t)units * kSliceMax) * 8 : 0;
   const int64_t ws_need = tile_bytes > cell_bytes ? tile_bytes : cell_bytes;
-  // fp8 copies of a pre-RoPE cache run the tile grids after the raw frames, on the same stream,
-  // with their tile maxima at the workspace's start (the raw append is done with it by then)
+  // fp8 copies of a pre-RoPE cache: chunks of few units form them with the raw frames, with both
+  // sets of tile maxima in the workspace (joint_bytes); otherwise (many units, or a caller's workspace
+  // of less than the size reported) the copies run the tile grids after the raw frames, on the same
+  // stream, with their tile maxima at the workspace's start (the raw append is done with it by then)
   const int copy_units = fp8 && kr_pool ? n_frames * batch * heads * (vr_pool ? 2 : 1) : 0;
   const int64_t copy_bytes = (int64_t)copy_units * a.ntiles * (int64_t)sizeof(float);
+  const int64_t joint_bytes = few_units && copy_units > 0 ? 2 * tile_bytes : 0;
   if (ws_query) {
-    *ws_query = ws_need > copy_bytes ? ws_need : copy_bytes;
+    *ws_query = std::max(ws_need, std::max(copy_bytes, joint_bytes));
     return SKV_OK;
   }
   if (copy_units > 0) {
@@ -1375,11 +1379,11 @@ static int append_impl(const void* k_new, const void* v_new, int src_dtype, int6
   }
   hipStream_t s = static_cast<hipStream_t>(stream);
   // Chunks of few units with copies: raw frames and copies together on the tile grids (two launches
-  // and two reads of the source, instead of the raw append's two and the copies' two), while both
-  // sets of tile maxima fit the workspace (frames of up to 4096 tokens with the size reported).
+  // and two reads of the source, instead of the raw append's two and the copies' two).
   // RoPE copy, same box: one frame of H24 x 880 tokens 23.0 -> 16.1 us; 3 frames, 4 streams, H12 x
-  // 1560 91.0 -> 73.7 us (with K norm 106.5 -> 76.9); PRoPE copies there 124.6 -> 91.7 us.
-  if (tile_split && copy_units > 0 && 2 * tile_bytes <= workspace_bytes) {
+  // 1560 91.0 -> 73.7 us (with K norm 106.5 -> 76.9); PRoPE copies there 124.6 -> 91.7 us.  Frames of
+  // 4480 to 16320 tokens take the same time either way (within 0.7%).
+  if (tile_split && copy_units > 0 && joint_bytes <= workspace_bytes) {
     float *part = static_cast<float*>(workspace), *part_x = part + (int64_t)units * a.ntiles;
     launch_fp8_both(a, src_dtype, dim3(units * a.ntiles), part, part_x, s);
     return launch_status();

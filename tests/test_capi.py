@@ -341,6 +341,8 @@ def test_fp8_copy_workspace_and_arguments():
         assert lib.skv_append_workspace_size(ctypes.byref(d), ctypes.byref(out)) == _lib.SKV_OK
         return out.value
 
+    # long frames of few units: raw frames and copies together, two floats per tile of the 12 units
+    assert need(desc(1, 2, 8960, 70)) == need(desc(1, 2, 8960, 70, prope=True)) == 2 * 12 * 140 * 4
     # 2304 raw units fill the chip (no raw workspace); the K copy: 3 x 16 x 24 units x 25 tiles
     assert need(desc(16, 24, 1560, 30)) == 3 * 16 * 24 * 25 * 4
     assert need(desc(16, 24, 1560, 30, prope=True)) == 2 * 3 * 16 * 24 * 25 * 4
