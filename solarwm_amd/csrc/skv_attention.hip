@@ -2644,8 +2644,8 @@ static int attention_impl(const void* q, int q_dtype, int64_t q_sb, int64_t q_st
   const int nt = a.nt;
   const int64_t qt8 = (int64_t)((q_len + kSplitBQ - 1) / kSplitBQ) * heads * batch;
   const int64_t units8 = qt8 * nt;
+  const int64_t unit_limit = (int64_t)1 << 31;  // share_begin counts a split's units in 32 bits
   if (mask_mode == SKV_MASK_NONE && n_segments == 0 && nt >= 8 && units8 >= 4 * n_cu &&
-      units8 < ((int64_t)1 << 31) &&
       n_cu <= kMaxSplitWg) {
     auto t_tile = [&](int64_t busy) { return 1.0 + 0.62 * (double)busy / n_cu; };
     auto t_grid = [&](int64_t wg, int per_cu, double per_tile) {  // rounds of nt tiles
@@ -2654,7 +2654,7 @@ static int attention_impl(const void* q, int q_dtype, int64_t q_sb, int64_t q_st
     };
     const double t_plain = nw == 8 ? t_grid(a.n_wg, 1, 1.0) : t_grid(a.n_wg, 2, 1.10);
     const double t_split = ((double)units8 / n_cu + 3.0) * t_tile(n_cu);
-    if (t_split < (nw == 8 ? 0.85 : 0.97) * t_plain) {
+    if (units8 < unit_limit && t_split < (nw == 8 ? 0.85 : 0.97) * t_plain) {
       split_bytes = split_workspace_bytes(n_cu);
       split_mode = 1;
     } else if (nw == 8 && a.n_wg > n_cu && a.n_wg % n_cu != 0) {
@@ -2662,7 +2662,7 @@ static int attention_impl(const void* q, int q_dtype, int64_t q_sb, int64_t q_st
       // share all CUs (C5: 912 q-tiles = 3 rounds + 144; the 4th round would run at 56% fill)
       const int64_t full = a.n_wg / n_cu, last = a.n_wg - full * n_cu;
       const double t_tail = full * nt * t_tile(n_cu) + ((double)last * nt / n_cu + 3.0) * t_tile(n_cu);
-      if (t_tail < 0.97 * t_plain) {
+      if (last * nt < unit_limit && t_tail < 0.97 * t_plain) {
         split_bytes = split_workspace_bytes(n_cu);
         split_mode = 2;
       }

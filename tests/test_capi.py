@@ -254,6 +254,18 @@ def test_launch_plans_of_benchmark_shapes(name, B, H, Lq, T, nf, pool, want):
         assert b"aligned" in lib.skv_last_error()
 
 
+def test_tail_split_counts_only_its_own_units():
+    """A grid of 2^31 (q-tile, key tile) pairs or more still splits its last round, whose own pairs are
+    what the shares count in 32 bits."""
+    for q_tiles, frames, want in ((300, 200, 1), (300, 220, 2), (511, 300, 0)):
+        d, _keep = _attn_desc(1, 1, 256 * q_tiles, 1 << 21, min(frames, 256))
+        d.workspace, d.workspace_bytes = 0x2000, SPLIT_BYTES
+        plan = _plan(d)
+        units = plan.n_qtiles * plan.key_tiles
+        assert (units < 2 ** 31) == (want == 1)
+        assert plan.split == want, (q_tiles, frames, plan.split)
+
+
 @pytest.mark.parametrize("name,B,H,Lq,T,nf,pool,want", [
     # 64-key tiles per query tile: packed across frame boundaries for whole bf16 / f16 frames of
     # T = 8k tokens (T not a multiple of 64), frame-aligned otherwise
