@@ -75,7 +75,8 @@ struct AttnArgs {
   const float* rope_hw;
   const float* rope_t;
   int gh, gw, n_qframes;
-  int rope_lds;  // 1: the kernels may stage rope_t in LDS per key frame (frames of >= 64 tokens)
+  int rope_lds;  // 1: the kernels may stage rope_t in LDS per key frame (frames of >= 64 tokens, 16-byte
+                 // aligned table)
   // PRoPE (camera transforms, applied after RoPE) on the same path; every matrix is a row-major
   // 4x4 acting on one group of 4 consecutive head channels:
   //   pq_t [B][n_frames][n_qframes][11][16]: W = R_k^T (P_q P_k^-1)^T R_q per temporal group
@@ -606,8 +607,8 @@ constexpr size_t attn_lds_bytes(int nw, int rm, int kt_bytes) {
          (rm == 1 && kt_bytes == 2 ? (size_t)attn_ring(nw, kt_bytes) * kTabSlot : 0);
 }
 
-// RM: 0 = Q as given, 1 = RoPE on load, 2 = RoPE + PRoPE, 3 = RoPE on load over frames of fewer than
-// 64 tokens.
+// RM: 0 = Q as given, 1 = RoPE on load, 2 = RoPE + PRoPE, 3 = RoPE on load with the angles straight
+// from memory (AttnArgs::rope_lds = 0).
 // PK: key tiles packed across frame boundaries (PackedWalk; whole frames of T = 8k tokens, 2-byte
 // pools, no RoPE): a window of n frames takes ceil(n T / 64) tiles instead of n ceil(T / 64).
 // SEG: the grid's q-tiles belong to consecutive query segments, each over its own slice of the
@@ -627,8 +628,8 @@ void attn_kernel(AttnArgs args) {
   constexpr int kRing = attn_ring(NW, (int)sizeof(KT));
   constexpr int kL = kRing / 2;
   constexpr int kWN = attn_wbufs(kRing);
-  // RoPE on load: the temporal angles come from LDS (RM = 1 over 2-byte pools) or, for frames under
-  // 64 tokens, straight from memory (RM = 3, and RM = 1 over fp8 pools)
+  // RoPE on load: the temporal angles come from LDS (RM = 1 over 2-byte pools) or straight from memory
+  // (RM = 3, and RM = 1 over fp8 pools of frames under 64 tokens)
   constexpr bool kRopeLds = RM == 1 && sizeof(KT) == 2;
   using ET = typename OpOf<KT>::E;     // MFMA operand element
   using etx8 = typename OpOf<KT>::x8;
@@ -2556,8 +2557,9 @@ static int attention_impl(const void* q, int q_dtype, int64_t q_sb, int64_t q_st
   a.q_rms = q_inv_rms;
   a.q_rms_sb = q_rms_sb;
   a.q_w = q_norm_weight;
-  // shorter frames would put more than kTabFrames query frames into a q-tile; the offsets are 32-bit
-  a.rope_lds = rope && frame_tokens >= kTile &&
+  // shorter frames would put more than kTabFrames query frames into a q-tile; the offsets are 32-bit;
+  // the pieces are 16 bytes, and a table may start at any float (its rows, 176 B, keep the alignment)
+  a.rope_lds = rope && frame_tokens >= kTile && reinterpret_cast<uintptr_t>(rope_t) % 16 == 0 &&
                (int64_t)n_qframes * n_frames * 8 * kRopeT < ((int64_t)1 << 31);
   a.gh = grid_h;
   a.gw = grid_w;

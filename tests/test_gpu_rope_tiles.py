@@ -56,6 +56,35 @@ def test_rope_on_load_edges(gpu, gh, gw, n, nq, H, dtype, norm, split):
         assert_attn_close(out, want)
 
 
+@pytest.mark.parametrize("norm,split", [(False, False), (True, True)])
+def test_rope_table_at_any_float(gpu, norm, split):
+    """A temporal table that starts 4, 8 or 12 bytes past a 16-byte boundary (a contiguous slice of a
+    larger tensor) gives what an aligned one gives: the instance that reads it from memory does the
+    same arithmetic, up to contractions in the query's float32 turn (bf16 rounding of the turned query
+    and of P: 2^-9 relative each)."""
+    gh, gw, n, nq, H = 8, 9, 40, 4, 7 if split else 2
+    T = gh * gw
+    g = torch.Generator(device=gpu).manual_seed(1)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=gpu)  # noqa: E731
+    q, w = rnd(1, nq * T, H, 128).bfloat16(), torch.rand(H * 128, generator=g, device=gpu) + 0.5
+    k, v = rnd(1, n * T, H, 128).bfloat16(), rnd(1, n * T, H, 128).bfloat16()
+    cfg = rope.RopeConfig(grid_hw=(gh, gw))
+    hw, tt = rope.spatial_table(cfg, gpu), rope.temporal_table(range(n - nq, n), range(n), cfg, gpu)
+    kp, vp, _, _ = kernels.new_pools(n, 1, H, T, torch.bfloat16, gpu)
+    krp = torch.zeros_like(kp)
+    kernels.append_frames(k, v, kp, vp, range(n), frame_tokens=T, kr_pool=krp, rope_hw=hw, grid_hw=(gh, gw))
+    kw = dict(frame_tokens=T, q_norm=(kernels.rms_rows(q, 1e-6), w) if norm else None)
+    assert (kernels.attention_plan(q, krp, vp, range(n), rope=(hw, (gh, gw), tt), **kw)["split"] == 1) == split
+    want = kernels.attention_frames(q, krp, vp, range(n), rope=(hw, (gh, gw), tt), **kw).float()
+    big = torch.empty(tt.numel() + 4, device=gpu)
+    assert tt.data_ptr() % 16 == 0 and big.data_ptr() % 16 == 0
+    for off in (1, 2, 3):
+        moved = big[off : off + tt.numel()].view(tt.shape)
+        moved.copy_(tt)
+        got = kernels.attention_frames(q, krp, vp, range(n), rope=(hw, (gh, gw), moved), **kw).float()
+        assert float((got - want).norm()) <= 2.0 ** -8 * float(want.norm()), off
+
+
 @pytest.mark.parametrize("H,Lq,T,n,dtype", [
     (1, 257 * 256 - 100, 64, 8, torch.bfloat16),    # 1 tail q-tile, 8 units over every CU: empty shares
     (3, 86 * 256, 72, 8, torch.float32),            # 2 tail q-tiles of 9 packed tiles
