@@ -2670,6 +2670,8 @@ static int attention_impl(const void* q, int q_dtype, int64_t q_sb, int64_t q_st
       }
     }
   }
+  // fp8 pools on the fp8 matrix cores (the others decode to bf16)
+  const bool mfma8 = pool_dtype == SKV_FP8_E4M3 && !prope && !(rope && frame_tokens < kTile);
   // Shares of a split over n_q q-tiles: one per CU, or, when they are not much longer for it, as
   // many as divide every q-tile evenly, so that no share crosses from one q-tile into the next.
   // A share that does pays a second start (query, first tiles) and a second record: some 8 us a
@@ -2682,21 +2684,36 @@ static int attention_impl(const void* q, int q_dtype, int64_t q_sb, int64_t q_st
   // -> 261.5, and RoPE, 96 x 294 (192, 37) 184 -> 191 a layer pass
   // (108 x 294, 216 shares, 23: 199 -> 196).  Tail launch of 60 q-tiles x 63 after three rounds: bf16
   // 452 -> 446, fp8 382 -> 368.
-  const bool mfma8 = pool_dtype == SKV_FP8_E4M3 && !prope && !(rope && frame_tokens < kTile);
   auto split_shares = [&](int64_t n_q) -> int {
     const int64_t m = n_cu / n_q, wg = m * n_q;
     return m >= 2 && (int64_t)nt * (n_cu - wg) <= (mfma8 ? 24 : 9) * m * n_cu ? (int)wg : n_cu;
   };
   // Unsplit grids that give every CU at most one workgroup either way: 4-wave groups spread the
-  // queries over twice the CUs and start sooner, which wins while the window is short (8 waves -> 4,
-  // us a launch: H24, 1215 queries x 512 keys 22.4 -> 17.4; H12, 1560 x 2048 50.7 -> 46.6; fp8 H24,
-  // 880 x 6160 99.5 -> 79.8; RoPE H12, 1760 x 98 tiles 136 -> 131); over long ones the 8-wave
-  // group's half as many staged bytes per query wins (H12, 1560 queries x 147 tiles 187 -> 191, x 512
-  // tiles 623 -> 648).  Up to 4 tiles they also win where they take two to a CU (H12, 4680 x 226 keys
-  // 18.7 -> 17.9; H16, 4000 x 77 16.4 -> 15.5; but 4680 x 512 keys 25.5 -> 26.9).
+  // queries over twice the CUs and start sooner (8 waves -> 4, us a launch; with a workspace, as the
+  // Python layer always passes one: H24, 1215 queries x 512 keys 22.4 -> 17.4; PRoPE H24, 1215 x 14
+  // tiles 33.0 -> 26.8; chunk-causal H4, 9 x 405 tokens 88.6 -> 75.6, H5, 6 x 1000 128.9 -> 122.6, fp8 103 ->
+  // 77).  Unmasked windows past some 15 tiles split, so only callers without a workspace come here with
+  // them: fp8 H24, 880 x 98 tiles 99.5 -> 79.8, RoPE H12, 1760 x 98 136 -> 131, bf16 H24, 1215 x 98 129
+  // -> 124, but H12, 1560 x 98 130 -> 133 and x 512 623 -> 648 (the 8-wave group stages half the bytes
+  // per query): up to 100 tiles; float32 pools, whose groups are bound by staging, up to 40 (H30, 256
+  // queries x 40 tiles even, x 70 213 -> 216).  2-byte windows past the 256 MB last-level cache lose:
+  // H110, 256 x 70 tiles (252 MB) 100.6 -> 103.6, H120 x 84 (330 MB) 124 -> 138, RoPE 138 -> 158, but
+  // H100 x 70 (229 MB) 98 -> 97.
+  // Windows of up to 4 tiles also win where 4-wave groups run two to a CU or in rounds (H12, 4680 x
+  // 226 keys 18.7 -> 17.9; H40, 6400 x 256 70 -> 64; but 4680 x 512 keys 25.5 -> 26.9).  Pools staged
+  // through registers lose there while the groups all run at once (float32 H64, 1024 x 256 keys 27.6
+  // -> 31.3, fp8 PRoPE H200, 210 x 70 keys 18.1 -> 18.8) and float32 ones with 3 or 4 tiles always
+  // (H40, 6400 x 256 102 -> 113; x 128, 25600 queries 356 -> 328).
   if (nw == 8 && n_segments == 0 && (split_bytes == 0 || workspace == nullptr)) {
     const int64_t wg4 = (int64_t)((q_len + 127) / 128) * heads * batch;
-    if (nt <= 4 || (nt <= 100 && wg4 <= n_cu)) {
+    const bool f32 = pool_dtype == SKV_F32;
+    const bool two_byte = pool_dtype == SKV_BF16 || pool_dtype == SKV_F16;
+    const bool reg_staged = f32 || (pool_dtype == SKV_FP8_E4M3 && !mfma8);
+    const int64_t window_bytes = (int64_t)batch * heads * nt * kTile * kHeadDim * 2 * 2;
+    const bool one_each = wg4 <= n_cu && nt <= (f32 && mask_mode == SKV_MASK_NONE ? 40 : 100) &&
+                          !(two_byte && window_bytes > (int64_t)224 << 20);
+    const bool few_tiles = nt <= (f32 ? 2 : 4) && !(reg_staged && wg4 <= 2 * n_cu);
+    if (one_each || few_tiles) {
       nw = 4;
       a.n_qtiles = (q_len + 127) / 128;
       a.n_wg = (int)wg4;

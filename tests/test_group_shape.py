@@ -21,6 +21,14 @@ from .test_capi import _attn_desc, _plan
     (1, 12, 4680, 256, 1, _lib.SKV_BF16, 4),    # 4 tiles
     (1, 12, 4680, 257, 1, _lib.SKV_BF16, 8),    # 5 tiles
     (1, 2, 128, 64, 5, _lib.SKV_FP8_E4M3, 4),
+    (1, 100, 256, 64, 70, _lib.SKV_BF16, 4),    # 200 groups over 229 MB of K and V
+    (1, 110, 256, 64, 70, _lib.SKV_BF16, 8),    # 252 MB
+    (1, 110, 256, 64, 70, _lib.SKV_FP8_E4M3, 4),
+    (1, 30, 256, 64, 40, _lib.SKV_F32, 4),      # float32 pools: up to 40 tiles
+    (1, 30, 256, 64, 41, _lib.SKV_F32, 8),
+    (1, 64, 1024, 64, 4, _lib.SKV_F32, 8),      # 512 groups: no short-window rule in one round
+    (1, 40, 25600, 64, 2, _lib.SKV_F32, 4),     # many rounds, 2 tiles
+    (1, 40, 25600, 64, 3, _lib.SKV_F32, 8),
 ])
 def test_waves_per_group(B, H, Lq, T, nf, pool, want):
     d, _keep = _attn_desc(B, H, Lq, T, nf, pool)
@@ -28,6 +36,22 @@ def test_waves_per_group(B, H, Lq, T, nf, pool, want):
     rows = 32 * want
     assert plan.waves_per_group == want and plan.split == 0
     assert plan.n_workgroups == plan.n_qtiles == -(-Lq // rows) * H * B
+
+
+def test_waves_per_group_of_other_launches():
+    """Chunk-causal float32 windows keep the longer line; fp8 frames decoded for PRoPE follow the
+    float32 rule while all groups run at once."""
+    d, _keep = _attn_desc(1, 4, 6016, 64, 94, _lib.SKV_F32, mask=_lib.SKV_MASK_CHUNK_CAUSAL)
+    assert _plan(d).waves_per_group == 4
+    for H, want in ((100, 4), (200, 8), (300, 4)):
+        d, _keep = _attn_desc(1, H, 192, 64, 2, _lib.SKV_FP8_E4M3)
+        fake = d.q
+        d.rope_hw, d.grid_h, d.grid_w, d.n_qframes = fake, 8, 8, 3
+        d.q_xform_t = d.q_xform_s = d.out_xform = fake
+        assert _plan(d).waves_per_group == want, H
+        d.q_xform_t = d.q_xform_s = d.out_xform = None
+        d.rope_t = fake  # on the fp8 matrix cores: 4 tiles and fewer on any grid
+        assert _plan(d).waves_per_group == 4
 
 
 @pytest.mark.gpu
