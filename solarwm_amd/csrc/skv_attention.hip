@@ -122,7 +122,12 @@ struct AttnArgs {
 // q-tiles of each XCD's last head ran alone at the end).  Dealt round-robin over the 8 XCDs, a
 // head's q-tiles stay on one XCD when the heads are a multiple of 8, and on two when of 4.  H24,
 // 21 x 405 tokens in chunks of 3 frames 562 -> 505 us a call; H12 355 -> 282; H12, 9 x 1560 907 ->
-// 765.  Grids of one round keep the plain order: the longest q-tile bounds them either way.
+// 765.  Other head counts, whose q-tiles meet every XCD, gain as much: H5, 12 x 1560 763 -> 515, H13,
+// 21 x 405 375 -> 284, H37, 12 x 405 336 -> 300; 4 streams of H40, 3 x 405 123 -> 117.  The plain order
+// stays for grids of one round (the longest q-tile bounds them either way) and, with at least as many
+// (stream, head) pairs as CUs (short sequences of a few q-tiles each), for 4-wave groups and float32
+// pools: 300 pairs, 8 x 80 tokens 77.1 -> 85.8, 4 x 80 36.9 -> 40.7, float32 4 x 300 388 -> 399 (but
+// 8-wave bf16 there 222 -> 209, and 200 pairs, 3 x 200 53.6 -> 52.0).
 __device__ inline void longest_first(const AttnArgs& a, int& qt, int& bh) {
   const int n_bh = a.B * a.H;
   qt = a.n_qtiles - 1 - (int)blockIdx.x / n_bh;
@@ -2745,7 +2750,8 @@ static int attention_impl(const void* q, int q_dtype, int64_t q_sb, int64_t q_st
   a.slot_stride = (int64_t)batch * heads * a.Tp * kHeadDim;
   a.scale_log2 = softmax_scale * 1.4426950408889634f;
   a.mask_mode = mask_mode;
-  a.by_length = mask_mode == SKV_MASK_CHUNK_CAUSAL && a.n_wg > n_cu * (8 / nw);
+  a.by_length = mask_mode == SKV_MASK_CHUNK_CAUSAL && a.n_wg > n_cu * (8 / nw) &&
+                !((int64_t)batch * heads >= n_cu && (nw == 4 || pool_dtype == SKV_F32));
   a.q_pos0 = q_pos0;
   a.chunk = chunk_tokens > 0 ? chunk_tokens : 1;
   a.n_keys = (int64_t)n_frames * frame_tokens;

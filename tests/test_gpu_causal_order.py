@@ -18,6 +18,8 @@ pytestmark = pytest.mark.gpu
     (2, 6, 6000, 777, torch.bfloat16),    # 24 x 12, chunk limits inside tiles
     (1, 37, 1801, 64, torch.float32),     # odd head count
     (3, 43, 400, 100, torch.bfloat16),    # 2 q-tiles x 129: the second round holds one workgroup
+    (1, 300, 320, 80, torch.bfloat16),    # as many heads as CUs, 4-wave groups: the plain order
+    (2, 150, 450, 60, torch.bfloat16),    # the same with 8-wave groups: longest first
 ])
 def test_longest_first_chunk_causal(gpu, B, H, L, chunk, dtype):
     print("causal order", B, H, L, chunk, dtype, flush=True)
