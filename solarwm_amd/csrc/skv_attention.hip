@@ -2675,8 +2675,6 @@ static int attention_impl(const void* q, int q_dtype, int64_t q_sb, int64_t q_st
       }
     }
   }
-  // fp8 pools on the fp8 matrix cores (the others decode to bf16)
-  const bool mfma8 = pool_dtype == SKV_FP8_E4M3 && !prope && !(rope && frame_tokens < kTile);
   // Shares of a split over n_q q-tiles: one per CU, or, when they are not much longer for it, as
   // many as divide every q-tile evenly, so that no share crosses from one q-tile into the next.
   // A share that does pays a second start (query, first tiles) and a second record: some 8 us a
@@ -2684,14 +2682,41 @@ static int attention_impl(const void* q, int q_dtype, int64_t q_sb, int64_t q_st
   // extra tiles, nt / m - n_q nt / n_cu.  One share a CU -> even shares, us a launch: bf16 H12,
   // 1560 queries x 147 tiles (84 q-tiles, 252 shares, 0.8 extra tiles) 117.4 -> 107.8; H24, 1215 x 126
   // (240 shares, 3.9) 136.4 -> 129.4; 44 q-tiles x 289 (220, 8.1) 141.4 -> 139.8; but 72 x 289 (216,
-  // 15) 210.7 -> 211.4 and 105 x 289 (210, 26) 291.9 -> 303.1.  fp8: H12, 1560 x 525 223 -> 205; 66 x
-  // 294 (198, 22) 145.7 -> 137.0; 105 x 294 (210, 26) 201.5 -> 197.3; but 95 x 525 (190, 68) 251.7
-  // -> 261.5, and RoPE, 96 x 294 (192, 37) 184 -> 191 a layer pass
-  // (108 x 294, 216 shares, 23: 199 -> 196).  Tail launch of 60 q-tiles x 63 after three rounds: bf16
-  // 452 -> 446, fp8 382 -> 368.
+  // 15) 210.7 -> 211.4 and 105 x 289 (210, 26) 291.9 -> 303.1.  Tail launch of 60 q-tiles x 63 after
+  // three rounds: bf16 452 -> 446, fp8 382 -> 368.
+  // The line (most extra tiles that still win) depends on what a tile costs, frame starts included
+  // (the query's turn, the scales, a short frame's padding), so on the instance and the tiles per
+  // frame, measured on 44 to 118 q-tiles (us at the q-tiles x tiles given, extra tiles in brackets):
+  //   bf16, f16  9; frames under 64 tokens 6: 95 x 60 [7.7] 71.7 -> 66.9, 118 x 230 [9] 258 -> 250;
+  //              48-token frames 66 x 119 [9] 99.5 -> 108.7, 110 x 71 [5] 94.9 -> 92.2
+  //   float32    5: 100 x 48 [5.2] 108.7 -> 106.5; 95 x 62 [8] 124.4 -> 128.6
+  //   RoPE       9; frames under 7 tiles 6: 7-tile 96 x 70 [8.8] 75.1 -> 70.7; 2-tile 100 x 82 [9] 104.2
+  //              -> 105.5, 118 x 128 [5] 168.9 -> 164.2; under 64 tokens 3 (fp8 too): 110 x 43 [3] 89.6
+  //              -> 87.8, 110 x 71 [5] 136.0 -> 139.8
+  //   PRoPE      9; under 7 tiles 5: 7-tile 104 x 98 [9.2] 103.7 -> 98.8; 2-tile 44 x 320 [9] 166.4 ->
+  //              170.0, 44 x 178 [5] 104.9 -> 97.1
+  //   fp8 PRoPE  9; under 14 tiles 5: 14-tile 108 x 112 [8.8] 125.5 -> 122.1; 7-tile 66 x 119 [9] 95.0 ->
+  //              97.5, 104 x 56 [5.2] 80.3 -> 76.8
+  //   fp8        24; under 7 tiles 17; one tile 10: 14-tile 108 x 294 [23] 167.1 -> 159.7; 2-tile 105 x
+  //              256 [23] 179.4 -> 186.6, 110 x 242 [17] 181.4 -> 178.7; 1-tile 105 x 167 [15] 143.9 ->
+  //              147.9, 110 x 128 [9] 126.6 -> 123.0
+  //   fp8 RoPE   22; under 14 tiles 16; under 7 tiles 4: 14-tile 108 x 224 [17.5] 141.6 -> 139.3; 7-tile
+  //              96 x 182 [23] 124.3 -> 127.3, 104 x 182 [17] 131.2 -> 128.9; 2-tile 105 x 156 [14] 155.6 ->
+  //              169.3, 118 x 128 [5] 146.2 -> 146.7, 95 x 38 [4.9] 70.6 -> 59.4
+  const int tiles_f = a.ntiles_f;
+  const bool fp8_pool = pool_dtype == SKV_FP8_E4M3, under64 = frame_tokens < kTile;
+  const int extra_tiles = prope         ? (tiles_f >= (fp8_pool ? 14 : 7) ? 9 : 5)
+                          : rope        ? (under64         ? 3
+                                           : !fp8_pool     ? (tiles_f >= 7 ? 9 : 6)
+                                           : tiles_f >= 14 ? 22
+                                           : tiles_f >= 7  ? 16
+                                                           : 4)
+                          : fp8_pool    ? (tiles_f >= 7 ? 24 : tiles_f >= 2 ? 17 : 10)
+                          : pool_dtype == SKV_F32 ? 5
+                                        : (under64 ? 6 : 9);
   auto split_shares = [&](int64_t n_q) -> int {
     const int64_t m = n_cu / n_q, wg = m * n_q;
-    return m >= 2 && (int64_t)nt * (n_cu - wg) <= (mfma8 ? 24 : 9) * m * n_cu ? (int)wg : n_cu;
+    return m >= 2 && (int64_t)nt * (n_cu - wg) <= extra_tiles * m * n_cu ? (int)wg : n_cu;
   };
   // Unsplit grids that give every CU at most one workgroup either way: 4-wave groups spread the
   // queries over twice the CUs and start sooner (8 waves -> 4, us a launch; with a workspace, as the
@@ -2713,7 +2738,8 @@ static int attention_impl(const void* q, int q_dtype, int64_t q_sb, int64_t q_st
     const int64_t wg4 = (int64_t)((q_len + 127) / 128) * heads * batch;
     const bool f32 = pool_dtype == SKV_F32;
     const bool two_byte = pool_dtype == SKV_BF16 || pool_dtype == SKV_F16;
-    const bool reg_staged = f32 || (pool_dtype == SKV_FP8_E4M3 && !mfma8);
+    // fp8 frames the fp8 matrix cores do not take are decoded to bf16
+    const bool reg_staged = f32 || (fp8_pool && (prope || (rope && under64)));
     const int64_t window_bytes = (int64_t)batch * heads * nt * kTile * kHeadDim * 2 * 2;
     const bool one_each = wg4 <= n_cu && nt <= (f32 && mask_mode == SKV_MASK_NONE ? 40 : 100) &&
                           !(two_byte && window_bytes > (int64_t)224 << 20);

@@ -3,10 +3,12 @@ grid the plan still reports) against float64 attention and the unsplit launch: 2
 q-tile, counts on both sides of the rule's line, bf16 / fp8 pools, float32 queries, a ragged last q-tile
 and the shares of a tail launch.  Bars: tests/helpers.py."""
 
+import ctypes
+
 import pytest
 import torch
 
-from solarwm_amd import kernels
+from solarwm_amd import _lib, kernels, rope
 
 from .helpers import assert_attn_close
 
@@ -54,3 +56,60 @@ def test_even_shares(gpu, H, Lq, T, n, pool, split, qt):
         for h in range(0, H, 7):  # every 7th head, one at a time: q-tiles of every share pattern
             want = torch.softmax(q64[h] @ k64[h].T / 128 ** 0.5, -1) @ v64[h]
             assert_attn_close(out[0, :, h], want.cpu())
+
+
+def _instance(gpu, mode, pool, H, T, n, nq):
+    """Random pools, query and tables of one attention instance; (query, K, V, kwargs)."""
+    g = torch.Generator(device=gpu).manual_seed(H + n)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=gpu)  # noqa: E731
+    tp = kernels.padded_tokens(T)
+    k, v = rnd(n, 1, H, tp, 128).to(pool), rnd(n, 1, H, 128, tp).to(pool)
+    kw = dict(frame_tokens=T)
+    if pool == F8:
+        kw |= dict(kscale=torch.full((n, 1, H), 0.5, device=gpu), vscale=torch.full((n, 1, H), 0.5, device=gpu))
+    if mode:
+        gh = next(x for x in range(int(T ** 0.5), 0, -1) if T % x == 0)
+        grid, eye = (gh, T // gh), torch.eye(4, device=gpu)
+        hw = rope.spatial_table(rope.RopeConfig(grid_hw=grid), gpu)
+        if mode == "rope":
+            kw["rope"] = (hw, grid, rope.temporal_table(range(n - nq, n), range(n), rope.RopeConfig(grid_hw=grid), gpu))
+        else:
+            kw["prope"] = (hw, grid, *(eye + 0.1 * rnd(*s, 4, 4) for s in ((1, n, nq, 11), (1, nq), (1, nq))))
+    return rnd(1, nq * T, H, 128).to(BF), k, v, kw
+
+
+@pytest.mark.parametrize("mode,pool,T,nq,even,uneven", [
+    ("", BF, 48, 5, 39, 60),              # 95 q-tiles: 190 even shares cost nt * 0.129 extra tiles
+    ("", torch.float32, 128, 2, 19, 24),
+    ("rope", BF, 128, 2, 22, 26),
+    ("rope", BF, 48, 5, 22, 39),
+    ("rope", F8, 128, 2, 15, 18),
+    ("rope", F8, 448, 1, 17, 20),
+    ("prope", BF, 128, 2, 19, 22),
+    ("prope", F8, 448, 1, 5, 6),
+    ("", F8, 64, 4, 74, 84),
+    ("", F8, 128, 2, 64, 70),
+])
+def test_share_count_follows_the_instance(gpu, mode, pool, T, nq, even, uneven):
+    """Workgroups that write records (the workspace starts as NaN), at frame counts on both sides of
+    the instance's line, and the result against the unsplit launch (bounds of test_even_shares)."""
+    H = 95 if T < 256 else 48  # 448-token queries take two q-tiles a head: 96
+    n_q = H * -(-nq * T // 256)
+    for n, want in ((even, 256 // n_q * n_q), (uneven, 256)):
+        print("share count", mode, pool, T, n, flush=True)
+        q, k, v, kw = _instance(gpu, mode, pool, H, T, n, nq)
+        plain = kernels.attention_frames(q, k, v, range(n), use_workspace=False, **kw)
+        d, out, keep = kernels.attention_desc(q, k, v, range(n), **kw)
+        plan = _lib.LaunchPlan()
+        lib = _lib.load()
+        _lib.check("plan", lib.skv_attention_plan(ctypes.byref(d), ctypes.byref(plan)))
+        n_cu = kernels.cu_count(gpu)
+        ws = torch.full((plan.workspace_bytes // 4,), float("nan"), device=gpu)
+        d.workspace, d.workspace_bytes = ws.data_ptr(), plan.workspace_bytes
+        _lib.check("attention", lib.skv_attention_ex(ctypes.byref(d), torch.cuda.current_stream().cuda_stream))
+        torch.cuda.synchronize()
+        ml = ws[2 * n_cu * 256 * 128 :].view(n_cu, 2, 256, 2)
+        wrote = (~ml[..., 0].isnan()).flatten(1).any(1)
+        assert int(wrote.sum()) == want, (n, int(wrote.sum()))
+        diff = (out.float() - plain.float()).norm() / plain.float().norm()
+        assert diff <= (3.8e-2 if pool == F8 and mode != "prope" else 4e-3), diff
