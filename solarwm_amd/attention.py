@@ -70,9 +70,8 @@ def attention(
         raise ValueError("q, k, v must be [B, L, H, D] with matching B, H and k.shape == v.shape")
     # attention.py:69-87: inputs that are not half precision are cast to `dtype`, then q and k
     # to v's dtype, and the kernel computes in that dtype.  bf16 runs the bf16 MFMA kernel (fp32
-    # inputs with dtype=bfloat16 are passed as fp32 and rounded to bf16 on load, the same
-    # rounding; K and V are rounded once, when they are staged); fp16 runs the same kernel on fp16
-    # pools with fp16 MFMAs.
+    # inputs with dtype=bfloat16 are passed as fp32 and rounded to bf16, the same rounding: Q on load,
+    # K and V when they are staged); fp16 runs the same kernel on fp16 pools with fp16 MFMAs.
     half = (torch.float16, torch.bfloat16)
 
     def to_half(x):
@@ -82,7 +81,7 @@ def attention(
         vh = to_half(v)
         kv_dtype = vh.dtype
         qh, kh = to_half(q).to(kv_dtype), to_half(k).to(kv_dtype)
-    else:  # fp32 inputs, dtype=bfloat16: the kernels round them to bf16 on load
+    else:  # fp32 inputs, dtype=bfloat16: the kernels round them to bf16
         kv_dtype = v.dtype
         qh, kh, vh = q.to(kv_dtype), k.to(kv_dtype), v
     if q_scale is not None:

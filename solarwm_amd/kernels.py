@@ -398,7 +398,7 @@ def stage_frames(k: torch.Tensor, v: torch.Tensor, n_frames: int, frame_tokens: 
         kpool, vpool = staging_pools(n_frames, b, h, frame_tokens, k.dtype, k.device)
         append_frames(k, v, kpool, vpool, list(range(n_frames)), frame_tokens=frame_tokens)
         return kpool, vpool
-    kpool, vpool = staging_pools(n_frames, b, h, frame_tokens, torch.bfloat16, k.device)
+    kpool, vpool = staging_pools(n_frames, b, h, frame_tokens, torch.bfloat16, k.device, k.dtype)
     launch = prepare_append(k, v, kpool, vpool, list(range(n_frames)), frame_tokens=frame_tokens,
                             entry="skv_append_round")
     launch()
@@ -683,7 +683,7 @@ def new_pools(
     return kpool, vpool, kscale, vscale
 
 
-_staging: dict[tuple[int, int, torch.dtype], torch.Tensor] = {}
+_staging: dict[tuple[int, int, torch.dtype, torch.dtype], torch.Tensor] = {}
 
 
 def staging_pools(
@@ -693,10 +693,13 @@ def staging_pools(
     frame_tokens: int,
     dtype: torch.dtype,
     device: torch.device,
+    source: torch.dtype | None = None,
 ) -> tuple[torch.Tensor, torch.Tensor]:
     """K/V pools of ``n_slots`` frames over this device and current stream's staging buffer, for
     dense K/V that a call stages and attends at once (the drop-in ``attention``, teacher
-    forcing).  The buffer grows on demand and is reused by every such call on the stream; its
+    forcing); ``source`` is the staged tensors' dtype where it is not the pools' (float32 values
+    rounded to bf16), and each (pool, source) pair has a buffer of its own, so calls of different
+    input types never share one.  The buffer grows on demand and is reused by every such call on the stream; its
     contents are left as they are (not zero-filled): an append writes every row of the slots it
     fills, rows past ``frame_tokens`` as zeros.  Calls on one stream run in order, so a call's
     append waits for the previous call's attention; the buffer stays allocated at its largest
@@ -705,7 +708,7 @@ def staging_pools(
         raise ValueError("staging pools hold bf16, f16 or float32 frames")
     tp = padded_tokens(frame_tokens)
     n = n_slots * batch * heads * tp * HEAD_DIM
-    key = (_device_index(device), _stream(device), dtype)
+    key = (_device_index(device), _stream(device), dtype, source or dtype)
     buf = _staging.get(key)
     if buf is None or buf.numel() < 2 * n:
         buf = torch.empty(2 * n, dtype=dtype, device=device)

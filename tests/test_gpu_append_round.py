@@ -24,7 +24,7 @@ def test_rounded_pools_bit_exact(gpu, B, H, T, n):
                         device=gpu)
     big[:, :, : n * T, :, 8:16] = edge
     k, v = big[0, ..., :128], big[1, ..., :128]
-    kernels.staging_pools(n, B, H, T, torch.bfloat16, gpu)[0].fill_(float("nan"))
+    kernels.staging_pools(n, B, H, T, torch.bfloat16, gpu, torch.float32)[0].fill_(float("nan"))
     kp, vp = kernels.stage_frames(k, v, n, T)
     kp, vp = kp.clone(), vp.clone()
     wk, wv, _, _ = kernels.new_pools(n, B, H, T, torch.bfloat16, gpu)
@@ -34,6 +34,17 @@ def test_rounded_pools_bit_exact(gpu, B, H, T, n):
         nan = want.isnan()
         assert torch.equal(got.isnan(), nan)
         assert torch.equal(got.view(torch.int16)[~nan], want.view(torch.int16)[~nan])
+
+
+def test_float32_and_bf16_calls_stage_apart(gpu):
+    """float32 K/V rounded to bf16 go to a buffer of their own: staging them leaves bf16 frames staged
+    on the same stream (by another thread, say) as they are."""
+    x = torch.randn(1, 64, 2, 128, device=gpu)
+    kp, vp = kernels.stage_frames(x.bfloat16(), x.bfloat16(), 1, 64)
+    before = kp.clone(), vp.clone()
+    kr, _ = kernels.stage_frames(x + 1, x + 1, 1, 64)
+    assert kr.data_ptr() != kp.data_ptr()
+    assert torch.equal(kp, before[0]) and torch.equal(vp, before[1])
 
 
 def test_round_refuses_other_types(gpu):
