@@ -92,9 +92,11 @@ def test_rope_table_at_any_float(gpu, norm, split):
 ])
 def test_merge_of_few_and_many_records(gpu, H, Lq, T, n, dtype):
     """The merge of split q-tiles where shares are empty, hold a single tile, or are many per
-    q-tile: against the unsplit launch of the same inputs, which differs by the order of the fp32
-    sums and one rounding to the output type (bf16: half an ulp of |x| <= 4 each side, 2 x 2^-7;
-    float32 outputs still carry P's bf16 rounding against another running max, 2^-9 relative)."""
+    q-tile: every row against the unsplit launch of the same inputs.  Both round P to bf16 against
+    another running max and, for bf16 outputs, the result: four roundings of rms 0.735 * 2^-7 /
+    sqrt(12) = 1.6e-3 relative, 3.1e-3 together.  A row is one draw over its keys and 128 channels, so
+    the bar is three times that, 1e-2 of the row's norm; a key tile lost or counted twice moves a row
+    by sqrt(1 / tiles), 0.11 at 80 tiles."""
     print("merge", H, Lq, T, n, dtype, flush=True)
     g = torch.Generator(device=gpu).manual_seed(H + n)
     rnd = lambda *s: torch.randn(*s, generator=g, device=gpu)  # noqa: E731
@@ -109,4 +111,5 @@ def test_merge_of_few_and_many_records(gpu, H, Lq, T, n, dtype):
     plain = kernels.attention_frames(q, kp, vp, slots, frame_tokens=T, use_workspace=False)
     torch.cuda.synchronize()
     assert torch.isfinite(out).all()
-    assert float((out.float() - plain.float()).abs().max()) <= 2.0 ** -6
+    moved = (out.float() - plain.float()).norm(dim=-1) / plain.float().norm(dim=-1)
+    assert float(moved.max()) <= 1e-2, float(moved.max())
