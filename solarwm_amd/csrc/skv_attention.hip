@@ -626,10 +626,10 @@ void attn_kernel(AttnArgs args) {
   static_assert(!SEG || (RM == 0 && !SPLIT), "segments: no RoPE, no split");
   constexpr int kBQ = NW * 32;
   // LDS map: kRing K buffers, then kRing V^T buffers (tile x in buffer x mod kRing), then (PRoPE)
-  // kWN matrix buffers.  A step reads K(tau+1) and V(tau-1) and loads K(tau+kL+1) and V(tau+kL-1);
-  // the workgroup meets at a barrier after every kL-th step.  kL = 1 (two buffers each) for
-  // 4-wave groups (two workgroups share a CU's LDS) and register-staged pools; the others take
-  // kL = 2.
+  // kWN matrix buffers or (RoPE, from LDS) kRing table slots.  A step reads K(tau+1) and V(tau-1) and
+  // loads K(tau+kL+1) and V(tau+kL-1); the workgroup meets at a barrier after every kL-th step.
+  // kL = 1 (two buffers each) for 4-wave groups (two workgroups share a CU's LDS) and register-staged
+  // pools; the others take kL = 2.
   constexpr int kRing = attn_ring(NW, (int)sizeof(KT));
   constexpr int kL = kRing / 2;
   constexpr int kWN = attn_wbufs(kRing);
@@ -638,7 +638,6 @@ void attn_kernel(AttnArgs args) {
   constexpr bool kRopeLds = RM == 1 && sizeof(KT) == 2;
   using ET = typename OpOf<KT>::E;     // MFMA operand element
   using etx8 = typename OpOf<KT>::x8;
-  // LDS: K tiles in [0, 32 KB) (two buffers), V^T tiles in [32 KB, 64 KB) (two buffers).
   extern __shared__ __attribute__((aligned(16))) char lds[];
   constexpr int kHalf = 16 * kBlockBytes;
 
@@ -722,8 +721,8 @@ void attn_kernel(AttnArgs args) {
   // behind lane-dependent branches (rows past the end, pairs that are temporal for one half of the
   // wave only) the RoPE / PRoPE instances waited out some thirty L2 round trips one by one at the
   // start of every q-tile (with the matrices read from LDS below: 30 layers of H24, 1215 queries
-  // over 18 x 405 keys, fused PRoPE, 5.74 -> 5.38 ms).  Rows past the end load the last row's, then count as zeros (their
-  // products then toggle few bits: at full chip the clock is power-limited).
+  // over 18 x 405 keys, fused PRoPE, 5.74 -> 5.38 ms).  Rows past the end load the last row's, then
+  // count as zeros (their products then toggle few bits: at full chip the clock is power-limited).
   const int qrc = min(qrow, qend - 1);
   [[maybe_unused]] int qfi = 0;  // query frame of this lane's row
   Vec8<QT> qx[8];
@@ -1335,7 +1334,6 @@ void attn_kernel(AttnArgs args) {
   static_assert(kL == 1 || kL == 2, "the barrier test above assumes kL <= 2 (cb = tau & 1)");
   int tau = 0;
   for (; tau + 1 < ntau; tau += 2) {
-
     step(tau, 0, sA, sB, pA, pB);
     step(tau + 1, 1, sB, sA, pB, pA);
   }
@@ -2058,7 +2056,6 @@ void attn_fp8_kernel(AttnArgs args) {
   };
   int tau = 0;
   for (; tau + 1 < ntau; tau += 2) {
-
     step(tau, 0, sA, sB, pA, pB);
     step(tau + 1, 1, sB, sA, pB, pA);
   }
