@@ -683,7 +683,7 @@ def new_pools(
     return kpool, vpool, kscale, vscale
 
 
-_staging: dict[tuple[int, int, torch.dtype, torch.dtype], torch.Tensor] = {}
+_staging: dict[tuple, torch.Tensor] = {}  # by (device, stream, pool dtype[, other source dtype])
 
 
 def staging_pools(
@@ -708,7 +708,9 @@ def staging_pools(
         raise ValueError("staging pools hold bf16, f16 or float32 frames")
     tp = padded_tokens(frame_tokens)
     n = n_slots * batch * heads * tp * HEAD_DIM
-    key = (_device_index(device), _stream(device), dtype, source or dtype)
+    key = (_device_index(device), _stream(device), dtype)
+    if source not in (None, dtype):
+        key += (source,)
     buf = _staging.get(key)
     if buf is None or buf.numel() < 2 * n:
         buf = torch.empty(2 * n, dtype=dtype, device=device)
