@@ -125,9 +125,10 @@ struct AttnArgs {
 // 765.  Other head counts, whose q-tiles meet every XCD, gain as much: H5, 12 x 1560 763 -> 515, H13,
 // 21 x 405 375 -> 284, H37, 12 x 405 336 -> 300; 4 streams of H40, 3 x 405 123 -> 117.  The plain order
 // stays for grids of one round (the longest q-tile bounds them either way) and, with at least as many
-// (stream, head) pairs as CUs (short sequences of a few q-tiles each), for 4-wave groups and float32
-// pools: 300 pairs, 8 x 80 tokens 77.1 -> 85.8, 4 x 80 36.9 -> 40.7, float32 4 x 300 388 -> 399 (but
-// 8-wave bf16 there 222 -> 209, and 200 pairs, 3 x 200 53.6 -> 52.0).
+// (stream, head) pairs as CUs (short sequences of a few q-tiles each), for 4-wave groups over 2-byte
+// pools and for float32 pools: 300 pairs, 8 x 80 tokens 77.1 -> 85.8, 4 x 80 36.9 -> 40.7, float32 400
+// pairs, 4 x 300 540 -> 611 (but 8-wave bf16, 300 pairs, 4 x 300 222 -> 209; fp8, 260 pairs, 8 x 80 67.7
+// -> 65.2; 200 pairs, 3 x 200 53.6 -> 52.0).
 __device__ inline void longest_first(const AttnArgs& a, int& qt, int& bh) {
   const int n_bh = a.B * a.H;
   qt = a.n_qtiles - 1 - (int)blockIdx.x / n_bh;
@@ -2684,33 +2685,40 @@ static int attention_impl(const void* q, int q_dtype, int64_t q_sb, int64_t q_st
   // The line (most extra tiles that still win) depends on what a tile costs, frame starts included
   // (the query's turn, the scales, a short frame's padding), so on the instance and the tiles per
   // frame, measured on 44 to 118 q-tiles (us at the q-tiles x tiles given, extra tiles in brackets):
-  //   bf16, f16  9; frames under 64 tokens 6: 95 x 60 [7.7] 71.7 -> 66.9, 118 x 230 [9] 258 -> 250;
-  //              48-token frames 66 x 119 [9] 99.5 -> 108.7, 110 x 71 [5] 94.9 -> 92.2
-  //   float32    5: 100 x 48 [5.2] 108.7 -> 106.5; 95 x 62 [8] 124.4 -> 128.6
-  //   RoPE       9; frames under 7 tiles 6: 7-tile 96 x 70 [8.8] 75.1 -> 70.7; 2-tile 100 x 82 [9] 104.2
-  //              -> 105.5, 118 x 128 [5] 168.9 -> 164.2; under 64 tokens 3 (fp8 too): 110 x 43 [3] 89.6
-  //              -> 87.8, 110 x 71 [5] 136.0 -> 139.8
-  //   PRoPE      9; under 7 tiles 5: 7-tile 104 x 98 [9.2] 103.7 -> 98.8; 2-tile 44 x 320 [9] 166.4 ->
-  //              170.0, 44 x 178 [5] 104.9 -> 97.1
-  //   fp8 PRoPE  9; under 14 tiles 5: 14-tile 108 x 112 [8.8] 125.5 -> 122.1; 7-tile 66 x 119 [9] 95.0 ->
-  //              97.5, 104 x 56 [5.2] 80.3 -> 76.8
-  //   fp8        24; under 7 tiles 17; one tile 10: 14-tile 108 x 294 [23] 167.1 -> 159.7; 2-tile 105 x
+  //   bf16, f16  9; frames under 64 tokens 7: 95 x 60 [7.7] 71.7 -> 66.9, 118 x 230 [9] 258 -> 250;
+  //              48-token frames 66 x 119 [9] 99.5 -> 108.7, 118 x 174 [6.8] 212.6 -> 209.8
+  //   float32    8: 72 x 116 [6] 162.5 -> 159.3, 118 x 204 [8] 394 -> 383, but 95 x 62 [8] 124.4 ->
+  //              128.6 and 44 x 284 [8] 218 -> 221
+  //   RoPE       9; one-tile frames 7: 2-tile 95 x 62 [8] 84.0 -> 80.3, 44 x 320 [9] 159.0 -> 160.8;
+  //              1-tile 72 x 134 [7] 127.1 -> 125.6; under 64 tokens 3 (fp8 too): 110 x 43 [3] 89.6 ->
+  //              87.8, 110 x 71 [5] 136.0 -> 139.8
+  //   PRoPE      9; one-tile frames 6: 2-tile 72 x 162 [8.4] 146.3 -> 141.2, 44 x 320 [9] 166.4 -> 170.0;
+  //              1-tile 118 x 128 [5] 197.8 -> 194.8
+  //   fp8 PRoPE  9; under 14 tiles 7; one tile 6: 14-tile 108 x 112 [8.8] 125.5 -> 122.1; 7-tile 66 x
+  //              119 [9] 95.0 -> 97.5, 104 x 77 [7.2] 97.2 -> 95.3; 2-tile 110 x 96 [6.8] 130.5 -> 128.0;
+  //              1-tile 95 x 41 [5.3] 82.2 -> 79.7
+  //   fp8        24; under 7 tiles 17; one tile 14: 14-tile 108 x 294 [23] 167.1 -> 159.7; 2-tile 105 x
   //              256 [23] 179.4 -> 186.6, 110 x 242 [17] 181.4 -> 178.7; 1-tile 105 x 167 [15] 143.9 ->
-  //              147.9, 110 x 128 [9] 126.6 -> 123.0
-  //   fp8 RoPE   22; under 14 tiles 16; under 7 tiles 4: 14-tile 108 x 224 [17.5] 141.6 -> 139.3; 7-tile
-  //              96 x 182 [23] 124.3 -> 127.3, 104 x 182 [17] 131.2 -> 128.9; 2-tile 105 x 156 [14] 155.6 ->
-  //              169.3, 118 x 128 [5] 146.2 -> 146.7, 95 x 38 [4.9] 70.6 -> 59.4
+  //              147.9, 95 x 116 [15] 110.9 -> 108.8, 100 x 110 [12] 111.3 -> 105.4
+  //   fp8 RoPE   22; under 14 tiles 17, 7 tiles 9, 3 tiles 6, one tile 5: 14-tile 108 x 224 [17.5] 141.6
+  //              -> 139.3; 7-tile 96 x 182 [23] 124.3 -> 127.3, 104 x 182 [17] 131.2 -> 128.9; 3-tile 118
+  //              x 129 [5] 130.2 -> 123.0; 2-tile 105 x 156 [14] 155.6 -> 169.3, 80 x 384 [8] 257 -> 266,
+  //              66 x 66 [5] 74.6 -> 67.2; 1-tile 118 x 128 [5] 187.2 -> 190.2, 100 x 46 [5] 90.2 -> 82.2
   const int tiles_f = a.ntiles_f;
   const bool fp8_pool = pool_dtype == SKV_FP8_E4M3, under64 = frame_tokens < kTile;
-  const int extra_tiles = prope         ? (tiles_f >= (fp8_pool ? 14 : 7) ? 9 : 5)
-                          : rope        ? (under64         ? 3
-                                           : !fp8_pool     ? (tiles_f >= 7 ? 9 : 6)
-                                           : tiles_f >= 14 ? 22
-                                           : tiles_f >= 7  ? 16
-                                                           : 4)
-                          : fp8_pool    ? (tiles_f >= 7 ? 24 : tiles_f >= 2 ? 17 : 10)
-                          : pool_dtype == SKV_F32 ? 5
-                                        : (under64 ? 6 : 9);
+  int extra_tiles;
+  if (prope)
+    extra_tiles = tiles_f == 1 ? 6 : fp8_pool && tiles_f < 14 ? 7 : 9;
+  else if (rope && under64)
+    extra_tiles = 3;
+  else if (rope && !fp8_pool)
+    extra_tiles = tiles_f == 1 ? 7 : 9;
+  else if (rope)
+    extra_tiles = tiles_f >= 14 ? 22 : tiles_f >= 7 ? 17 : tiles_f >= 3 ? 9 : tiles_f == 2 ? 6 : 5;
+  else if (fp8_pool)
+    extra_tiles = tiles_f >= 7 ? 24 : tiles_f >= 2 ? 17 : 14;
+  else
+    extra_tiles = pool_dtype == SKV_F32 ? 8 : under64 ? 7 : 9;
   auto split_shares = [&](int64_t n_q) -> int {
     const int64_t m = n_cu / n_q, wg = m * n_q;
     return m >= 2 && (int64_t)nt * (n_cu - wg) <= extra_tiles * m * n_cu ? (int)wg : n_cu;
@@ -2722,15 +2730,17 @@ static int attention_impl(const void* q, int q_dtype, int64_t q_sb, int64_t q_st
   // 77).  Unmasked windows past some 15 tiles split, so only callers without a workspace come here with
   // them: fp8 H24, 880 x 98 tiles 99.5 -> 79.8, RoPE H12, 1760 x 98 136 -> 131, bf16 H24, 1215 x 98 129
   // -> 124, but H12, 1560 x 98 130 -> 133 and x 512 623 -> 648 (the 8-wave group stages half the bytes
-  // per query): up to 100 tiles; float32 pools, whose groups are bound by staging, up to 40 (H30, 256
-  // queries x 40 tiles even, x 70 213 -> 216).  2-byte windows past the 256 MB last-level cache lose:
+  // per query): up to 100 tiles; float32 pools, whose groups are bound by staging, up to 40 where the
+  // 4-wave groups take less than half the CUs (H30, 256 queries x 40 tiles even, x 70 213 -> 216; but
+  // H90, 256 x 88 315.5 -> 302.8).  2-byte windows past the 256 MB last-level cache lose:
   // H110, 256 x 70 tiles (252 MB) 100.6 -> 103.6, H120 x 84 (330 MB) 124 -> 138, RoPE 138 -> 158, but
   // H100 x 70 (229 MB) 98 -> 97.
   // Windows of up to 4 tiles also win where 4-wave groups run two to a CU or in rounds (H12, 4680 x
   // 226 keys 18.7 -> 17.9; H40, 6400 x 256 70 -> 64; but 4680 x 512 keys 25.5 -> 26.9).  Pools staged
   // through registers lose there while the groups all run at once (float32 H64, 1024 x 256 keys 27.6
-  // -> 31.3, fp8 PRoPE H200, 210 x 70 keys 18.1 -> 18.8) and float32 ones with 3 or 4 tiles always
-  // (H40, 6400 x 256 102 -> 113; x 128, 25600 queries 356 -> 328).
+  // -> 31.3, fp8 PRoPE H200, 210 x 70 keys 18.1 -> 18.8), float32 ones of 3 or 4 tiles up to some twelve
+  // groups a CU (H40, 6400 x 256 102 -> 113, H256, 1360 x 4 tiles 165 -> 176; H128, 3400 x 4 227 -> 208,
+  // H256, 8000 x 4 1307 -> 886; x 128 keys, H40, 25600 queries 356 -> 328).
   if (nw == 8 && n_segments == 0 && (split_bytes == 0 || workspace == nullptr)) {
     const int64_t wg4 = (int64_t)((q_len + 127) / 128) * heads * batch;
     const bool f32 = pool_dtype == SKV_F32;
@@ -2738,9 +2748,10 @@ static int attention_impl(const void* q, int q_dtype, int64_t q_sb, int64_t q_st
     // fp8 frames the fp8 matrix cores do not take are decoded to bf16
     const bool reg_staged = f32 || (fp8_pool && (prope || (rope && under64)));
     const int64_t window_bytes = (int64_t)batch * heads * nt * kTile * kHeadDim * 2 * 2;
-    const bool one_each = wg4 <= n_cu && nt <= (f32 && mask_mode == SKV_MASK_NONE ? 40 : 100) &&
-                          !(two_byte && window_bytes > (int64_t)224 << 20);
-    const bool few_tiles = nt <= (f32 ? 2 : 4) && !(reg_staged && wg4 <= 2 * n_cu);
+    const bool one_each = wg4 <= n_cu && nt <= 100 &&
+                          !(two_byte && window_bytes > (int64_t)224 << 20) &&
+                          !(f32 && mask_mode == SKV_MASK_NONE && nt > 40 && 2 * wg4 < n_cu);
+    const bool few_tiles = nt <= 4 && !(reg_staged && wg4 <= (f32 && nt > 2 ? 12 : 2) * n_cu);
     if (one_each || few_tiles) {
       nw = 4;
       a.n_qtiles = (q_len + 127) / 128;
@@ -2774,7 +2785,8 @@ static int attention_impl(const void* q, int q_dtype, int64_t q_sb, int64_t q_st
   a.scale_log2 = softmax_scale * 1.4426950408889634f;
   a.mask_mode = mask_mode;
   a.by_length = mask_mode == SKV_MASK_CHUNK_CAUSAL && a.n_wg > n_cu * (8 / nw) &&
-                !((int64_t)batch * heads >= n_cu && (nw == 4 || pool_dtype == SKV_F32));
+                !((int64_t)batch * heads >= n_cu &&
+                  (pool_dtype == SKV_F32 || (nw == 4 && pool_dtype != SKV_FP8_E4M3)));
   a.q_pos0 = q_pos0;
   a.chunk = chunk_tokens > 0 ? chunk_tokens : 1;
   a.n_keys = (int64_t)n_frames * frame_tokens;

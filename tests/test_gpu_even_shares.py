@@ -79,15 +79,21 @@ def _instance(gpu, mode, pool, H, T, n, nq):
 
 
 @pytest.mark.parametrize("mode,pool,T,nq,even,uneven", [
-    ("", BF, 48, 5, 39, 60),              # 95 q-tiles: 190 even shares cost nt * 0.129 extra tiles
-    ("", torch.float32, 128, 2, 19, 24),
-    ("rope", BF, 128, 2, 22, 26),
+    ("", BF, 48, 5, 53, 60),              # 95 q-tiles: 190 even shares cost nt * 0.129 extra tiles
+    ("", BF, 64, 4, 69, 71),
+    ("", torch.float32, 128, 2, 31, 32),
+    ("rope", BF, 64, 4, 54, 55),
+    ("rope", BF, 128, 2, 34, 36),
     ("rope", BF, 48, 5, 22, 39),
-    ("rope", F8, 128, 2, 15, 18),
-    ("rope", F8, 448, 1, 17, 20),
-    ("prope", BF, 128, 2, 19, 22),
-    ("prope", F8, 448, 1, 5, 6),
-    ("", F8, 64, 4, 74, 84),
+    ("rope", F8, 64, 4, 38, 39),
+    ("rope", F8, 128, 2, 23, 24),
+    ("rope", F8, 192, 1, 23, 24),
+    ("rope", F8, 448, 1, 19, 20),         # 96 q-tiles: nt * 0.125
+    ("prope", BF, 64, 4, 46, 47),
+    ("prope", BF, 128, 2, 34, 36),
+    ("prope", F8, 128, 2, 27, 28),
+    ("prope", F8, 448, 1, 8, 9),
+    ("", F8, 64, 4, 108, 110),
     ("", F8, 128, 2, 64, 70),
 ])
 def test_share_count_follows_the_instance(gpu, mode, pool, T, nq, even, uneven):

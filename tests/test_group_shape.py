@@ -24,11 +24,15 @@ from .test_capi import _attn_desc, _plan
     (1, 100, 256, 64, 70, _lib.SKV_BF16, 4),    # 200 groups over 229 MB of K and V
     (1, 110, 256, 64, 70, _lib.SKV_BF16, 8),    # 252 MB
     (1, 110, 256, 64, 70, _lib.SKV_FP8_E4M3, 4),
-    (1, 30, 256, 64, 40, _lib.SKV_F32, 4),      # float32 pools: up to 40 tiles
+    (1, 30, 256, 64, 40, _lib.SKV_F32, 4),      # float32 pools: up to 40 tiles on under half the CUs
     (1, 30, 256, 64, 41, _lib.SKV_F32, 8),
+    (1, 63, 256, 64, 41, _lib.SKV_F32, 8),
+    (1, 64, 256, 64, 41, _lib.SKV_F32, 4),
     (1, 64, 1024, 64, 4, _lib.SKV_F32, 8),      # 512 groups: no short-window rule in one round
     (1, 40, 25600, 64, 2, _lib.SKV_F32, 4),     # many rounds, 2 tiles
-    (1, 40, 25600, 64, 3, _lib.SKV_F32, 8),
+    (1, 40, 6400, 64, 4, _lib.SKV_F32, 8),      # 3 or 4 tiles: 2000 groups
+    (1, 256, 1536, 64, 4, _lib.SKV_F32, 8),     # 3072
+    (1, 256, 1537, 64, 4, _lib.SKV_F32, 4),     # 3328
 ])
 def test_waves_per_group(B, H, Lq, T, nf, pool, want):
     d, _keep = _attn_desc(B, H, Lq, T, nf, pool)
