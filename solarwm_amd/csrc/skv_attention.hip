@@ -2700,10 +2700,10 @@ static int attention_impl(const void* q, int q_dtype, int64_t q_sb, int64_t q_st
   //   fp8        24; under 7 tiles 17; one tile 14: 14-tile 108 x 294 [23] 167.1 -> 159.7; 2-tile 105 x
   //              256 [23] 179.4 -> 186.6, 110 x 242 [17] 181.4 -> 178.7; 1-tile 105 x 167 [15] 143.9 ->
   //              147.9, 95 x 116 [15] 110.9 -> 108.8, 100 x 110 [12] 111.3 -> 105.4
-  //   fp8 RoPE   22; under 14 tiles 17, 7 tiles 9, 3 tiles 6, one tile 5: 14-tile 108 x 224 [17.5] 141.6
+  //   fp8 RoPE   22; under 14 tiles 17, 7 tiles 9, 3 tiles 6: 14-tile 108 x 224 [17.5] 141.6
   //              -> 139.3; 7-tile 96 x 182 [23] 124.3 -> 127.3, 104 x 182 [17] 131.2 -> 128.9; 3-tile 118
   //              x 129 [5] 130.2 -> 123.0; 2-tile 105 x 156 [14] 155.6 -> 169.3, 80 x 384 [8] 257 -> 266,
-  //              66 x 66 [5] 74.6 -> 67.2; 1-tile 118 x 128 [5] 187.2 -> 190.2, 100 x 46 [5] 90.2 -> 82.2
+  //              66 x 66 [5] 74.6 -> 67.2; 1-tile 118 x 128 [5] 187.2 -> 190.2, 66 x 69 [5.2] 90.2 -> 82.9
   const int tiles_f = a.ntiles_f;
   const bool fp8_pool = pool_dtype == SKV_FP8_E4M3, under64 = frame_tokens < kTile;
   int extra_tiles;
@@ -2714,7 +2714,7 @@ static int attention_impl(const void* q, int q_dtype, int64_t q_sb, int64_t q_st
   else if (rope && !fp8_pool)
     extra_tiles = tiles_f == 1 ? 7 : 9;
   else if (rope)
-    extra_tiles = tiles_f >= 14 ? 22 : tiles_f >= 7 ? 17 : tiles_f >= 3 ? 9 : tiles_f == 2 ? 6 : 5;
+    extra_tiles = tiles_f >= 14 ? 22 : tiles_f >= 7 ? 17 : tiles_f >= 3 ? 9 : 6;
   else if (fp8_pool)
     extra_tiles = tiles_f >= 7 ? 24 : tiles_f >= 2 ? 17 : 14;
   else

@@ -85,7 +85,7 @@ def _instance(gpu, mode, pool, H, T, n, nq):
     ("rope", BF, 64, 4, 54, 55),
     ("rope", BF, 128, 2, 34, 36),
     ("rope", BF, 48, 5, 22, 39),
-    ("rope", F8, 64, 4, 38, 39),
+    ("rope", F8, 64, 4, 46, 47),
     ("rope", F8, 128, 2, 23, 24),
     ("rope", F8, 192, 1, 23, 24),
     ("rope", F8, 448, 1, 19, 20),         # 96 q-tiles: nt * 0.125
